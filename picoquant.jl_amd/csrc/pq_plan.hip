@@ -40,11 +40,15 @@ namespace {
 // lanes, many outputs give 256 outputs one lane each): lane (b0, j) sums
 // entries b = b0, b0 + tb, ... of its output (the tj lanes of one b0 read
 // adjacent elements), then the tb partial sums of each output are added
-// pairwise in LDS.
+// pairwise in LDS.  One launch covers every output batch whose copies the
+// slice group holds.
 template <typename C>
 __global__ __launch_bounds__(256) void k_accum(const C* __restrict__ src, int64_t elems, int64_t stride, int nb,
                                                int log_tj, int overwrite, double* __restrict__ out) {
   __shared__ double pr[256], pi[256];
+  // grid y: the output batches of the slice group (nb copies each)
+  src += (int64_t)blockIdx.y * nb * stride;
+  out += (int64_t)blockIdx.y * 2 * elems;
   const int tj = 1 << log_tj, tb = 256 >> log_tj;
   const int lj = threadIdx.x & (tj - 1), b0 = threadIdx.x >> log_tj;
   const int64_t j = (int64_t)blockIdx.x * tj + lj;
@@ -169,6 +173,7 @@ struct pq_plan {
   const int32_t* f_lv = nullptr;
   size_t f_lds = 0;                  // forest launch: LDS bytes of the largest tree (0: none)
   int n_sliced = 0, group_bits = 0;
+  int out_in_group = 0;              // output-batch bonds the slice group covers (its highest bits)
   int64_t n_groups = 1;
   struct OutQubit {
     int slot, bit;                   // leaf slot of a closed output qubit, its bit in a bitstring word
@@ -798,45 +803,86 @@ int run_program(pq_ctx* c, pq_plan* p, bool profile_steps) {
     if (r) return r;
   }
   const Slot& os = p->slots[p->out_slot];
-  int nbatch = (int)os.copies();
+  const int nbatch = (int)(os.copies() >> p->out_in_group);   // slices summed per output batch
   for (int64_t grp = 0; grp < p->n_groups; ++grp) {
     {
       int r = run_seq(1, p->seq2, grp);
       if (r) return r;
     }
     const void* src = slot_ptr(c, p, p->out_slot, grp);
-    // the group's output batch: its bits above the summed slice bonds; the
-    // batch's first group writes it
-    const int summed = p->n_sliced - p->n_out_bits - p->group_bits;
-    double* dst = p->out_dev + 2 * p->out_elems * (grp >> summed);
+    // the group's output batches: its own 2^out_in_group, or the one named
+    // by its bits above the summed slice bonds; a batch's first group
+    // writes it
+    const int oig = p->out_in_group;
+    const int summed = p->n_sliced - p->n_out_bits - (p->group_bits - oig);
+    double* dst = p->out_dev + 2 * p->out_elems * ((grp >> summed) << oig);
     const int first = (grp & (((int64_t)1 << summed) - 1)) == 0 ? 1 : 0;
     const int lt = accum_log_tj(os.elems, nbatch);
     const unsigned ga = (unsigned)((os.elems + (1 << lt) - 1) >> lt);
-    ProfScope ps(c, PQ_KC_ACCUM, (double)os.elems * nbatch * esize_of(os.dtype) + 16.0 * os.elems, 0);
+    const double nout = (double)((int64_t)1 << oig);
+    ProfScope ps(c, PQ_KC_ACCUM, nout * ((double)os.elems * nbatch * esize_of(os.dtype) + 16.0 * os.elems), 0);
     if (os.dtype == PQ_C128)
-      hipLaunchKernelGGL((k_accum<c128>), dim3(ga), dim3(256), 0, c->stream, (const c128*)src,
+      hipLaunchKernelGGL((k_accum<c128>), dim3(ga, 1u << oig), dim3(256), 0, c->stream, (const c128*)src,
                          os.elems, os.elems, nbatch, lt, first, dst);
     else
-      hipLaunchKernelGGL((k_accum<c64>), dim3(ga), dim3(256), 0, c->stream, (const c64*)src,
+      hipLaunchKernelGGL((k_accum<c64>), dim3(ga, 1u << oig), dim3(256), 0, c->stream, (const c64*)src,
                          os.elems, os.elems, nbatch, lt, first, dst);
     if (hipGetLastError() != hipSuccess) return fail(c, PQ_ERR_HIP, "accumulate kernel");
   }
   return PQ_OK;
 }
 
-}  // namespace
+// Output-batch bonds that join the slice group: a batch of bitstrings then
+// runs as more copies of each batched step (grid z, or extra rows of a
+// product whose other operand no bitstring changes) instead of once more
+// through the launch sequence per bitstring.  A launch is worth the batch
+// while its tensors are small: 64 ComplexF64 amplitudes of the 5x5
+// depth-12 grid circuit (peak 2^18 elements) took 17.2 ms as 64 groups of
+// launches of 4-23 us each, and take 1.70 ms in one group.  The copies of
+// every intermediate stay within OUT_GROUP_BYTES, the size of the last-level
+// cache (16 / 64 / 1024 MiB on that plan: 6.23 / 2.67 / 1.69 ms; the limit
+// also keeps every stride far below 2^31), a group has at most
+// PQ_MAX_BMODES bits, and plans whose fused chains depend on the bitstrings
+// keep one group per bitstring (a chain runs once per group).
+#define OUT_GROUP_BYTES ((int64_t)256 << 20)
+int out_bits_in_group(const pq_ctx* c, const pq_plan_desc* d) {
+  if (d->n_slots <= 0 || d->n_steps < 0 || d->n_sliced < 0 || d->n_sliced > 40 || d->group_bits < 0 ||
+      d->n_out_bits < 1 || d->n_out_bits > d->n_sliced || d->group_bits != d->n_sliced - d->n_out_bits ||
+      !d->slot_batch_mask)
+    return 0;
+  if (d->step_kind)
+    for (int i = 0; i < d->n_steps; ++i) {
+      const int cs = d->step_slots[3 * i + 2];
+      if (d->step_kind[i] == 2 && cs >= 0 && cs < d->n_slots && ((uint64_t)d->slot_batch_mask[cs] >> d->group_bits))
+        return 0;
+    }
+  int e = std::min(d->n_out_bits, PQ_MAX_BMODES - d->group_bits);
+  for (; e > 0; --e) {
+    bool fits = true;
+    for (int s = 0; s < d->n_slots && fits; ++s) {
+      const uint64_t low = (uint64_t)d->slot_batch_mask[s] & (((uint64_t)1 << (d->group_bits + e)) - 1);
+      const int64_t es = (d->slot_dtype ? d->slot_dtype[s] : c->dtype) == PQ_C128 ? 16 : 8;
+      if (low >> d->group_bits)
+        fits = d->slot_elems[s] > 0 &&
+               d->slot_elems[s] <= (OUT_GROUP_BYTES / es) >> __builtin_popcountll(low);
+    }
+    if (fits) break;
+  }
+  return std::max(e, 0);
+}
 
-extern "C" {
-
-int pq_plan_create(pq_ctx* c, const pq_plan_desc* d, pq_plan** out) {
-  if (!c || !d || !out) return PQ_ERR_ARG;
+// Builds the plan with out_in_group of the output-batch bonds inside the
+// slice group.
+int create_plan(pq_ctx* c, const pq_plan_desc* d, int out_in_group, pq_plan** out) {
   if (d->n_slots <= 0 || d->n_steps < 0 || d->n_sliced < 0 || d->n_sliced > 40 || d->group_bits < 0 ||
       d->group_bits > d->n_sliced || d->group_bits > 16 || d->out_slot < 0 || d->out_slot >= d->n_slots)
     return fail(c, PQ_ERR_ARG, "bad plan header");
   pq_plan* p = new pq_plan;
   p->n_sliced = d->n_sliced;
-  p->group_bits = d->group_bits;
-  p->n_groups = (int64_t)1 << (d->n_sliced - d->group_bits);
+  const int group_bits = d->group_bits + out_in_group;
+  p->group_bits = group_bits;
+  p->out_in_group = out_in_group;
+  p->n_groups = (int64_t)1 << (d->n_sliced - group_bits);
   if (d->n_out_bits < 0 || d->n_out_bits > d->n_sliced - d->group_bits) {
     delete p;
     return fail(c, PQ_ERR_ARG, "output batch bonds must lie above the slice group");
@@ -855,7 +901,7 @@ int pq_plan_create(pq_ctx* c, const pq_plan_desc* d, pq_plan** out) {
     const uint64_t m = d->slot_batch_mask ? (uint64_t)d->slot_batch_mask[s] : 0;
     if (d->n_sliced < 64 && (m >> d->n_sliced) != 0) return bad("batch mask names a bond that is not sliced");
     sl.mask = m;
-    sl.low = m & (((uint64_t)1 << d->group_bits) - 1);
+    sl.low = m & (((uint64_t)1 << group_bits) - 1);
     sl.batched = m != 0;
     sl.leaf = d->slot_leaf[s];
     sl.dtype = d->slot_dtype ? d->slot_dtype[s] : c->dtype;
@@ -942,7 +988,7 @@ int pq_plan_create(pq_ctx* c, const pq_plan_desc* d, pq_plan** out) {
         if (m.ext < 1 || m.s0 < 0 || m.s1 < 0) return bad("bad mode");
     const Slot &A = p->slots[st.a], &B = p->slots[st.b], &Cs = p->slots[st.c];
     st.dep = Cs.batched;
-    st.phase2 = (Cs.mask >> d->group_bits) != 0;
+    st.phase2 = (Cs.mask >> group_bits) != 0;
     if ((A.mask | B.mask) & ~Cs.mask) return bad("result independent of a sliced bond its operand depends on");
     if (st.kind == 2) {
       const char* why = parse_chain(c, p, d, i, st, produced, chain_tab);
@@ -989,7 +1035,7 @@ int pq_plan_create(pq_ctx* c, const pq_plan_desc* d, pq_plan** out) {
         return sl.slice_stride[j];
       };
       L.nmodes = 0;
-      for (int j = 0; j < d->group_bits; ++j) {
+      for (int j = 0; j < group_bits; ++j) {
         if (!((Cs.low >> j) & 1)) continue;
         const int q = L.nmodes++;
         L.ext[q] = make_fdiv(2);
@@ -1245,7 +1291,7 @@ int pq_plan_create(pq_ctx* c, const pq_plan_desc* d, pq_plan** out) {
     return fail(c, PQ_ERR_OOM, "plan memory allocation failed");
   }
   // Grouped descriptors (pointers of slice group 0 + per-bit leaf offsets).
-  if (d->n_sliced - d->group_bits > PQ_MAX_HIGH_BITS) {
+  if (d->n_sliced - group_bits > PQ_MAX_HIGH_BITS) {
     bool any = false;
     for (auto* seq : {&p->seq1, &p->seq2})
       for (const Launch& L : *seq) any = any || L.grouped;
@@ -1288,9 +1334,9 @@ int pq_plan_create(pq_ctx* c, const pq_plan_desc* d, pq_plan** out) {
           maxw = std::max<uint64_t>(maxw, st.spec.Mt * st.spec.Nt);
           maxb = std::max<unsigned>(maxb, st.spec.L.total);
         }
-        m.nhigh = st.phase2 ? d->n_sliced - d->group_bits : 0;
+        m.nhigh = st.phase2 ? d->n_sliced - group_bits : 0;
         for (int j = 0; j < m.nhigh; ++j) {
-          const int bit = d->group_bits + j;
+          const int bit = group_bits + j;
           m.hA[j] = p->slots[st.a].slice_stride[bit];
           m.hB[j] = p->slots[st.b].slice_stride[bit];
           // a conversion's output keeps the same sliced bonds as its input
@@ -1554,6 +1600,19 @@ int pq_plan_create(pq_ctx* c, const pq_plan_desc* d, pq_plan** out) {
   }
   *out = p;
   return PQ_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int pq_plan_create(pq_ctx* c, const pq_plan_desc* d, pq_plan** out) {
+  if (!c || !d || !out) return PQ_ERR_ARG;
+  const int e = out_bits_in_group(c, d);
+  // a plan that cannot be built with its output batches in the slice group
+  // (memory, launch limits) runs them one after another
+  if (e > 0 && create_plan(c, d, e, out) == PQ_OK) return PQ_OK;
+  return create_plan(c, d, 0, out);
 }
 
 int pq_plan_execute(pq_ctx* c, pq_plan* p, int use_graph) {

@@ -181,3 +181,30 @@ def test_bad_bitstring_batches_are_rejected():
         compile_plan(tn, plan, bitstrings=["011"])           # too short
     with pytest.raises(ValueError):
         compile_plan(tn, plan, bitstrings=[])
+
+
+@pytest.mark.parametrize("n_sliced,group_bits,precision,count", [
+    (0, 0, "uniform", 1), (0, 0, "uniform", 2), (0, 0, "uniform", 37), (3, 3, "uniform", 5), (3, 3, "mixed", 16),
+    (8, 8, "uniform", 32), (3, 1, "uniform", 5)])
+def test_bitstring_batch_inside_the_slice_group(n_sliced, group_bits, precision, count):
+    """Every slice in one group: the batch's bitstrings join it as more copies
+    (13 bits with 8 slices' bonds and 32 bitstrings, one more than a group
+    holds, so two groups run); with slice groups left over (the last case)
+    they stay one group each.  Replays with rewritten batches, padded counts
+    and an open qubit, against brute force; FP64 as the plan executor's other
+    tests, mixed precision at its 1e-5."""
+    n = 12
+    sv = O.statevector(n, O.grid_circuit_gates(3, 4, 8, 5))
+    rng = np.random.default_rng(count + n_sliced)
+    batches = [["".join("x" if i == 7 else str(int(v)) for i, v in enumerate(rng.integers(0, 2, n)))
+                for _ in range(count)] for _ in range(2)]
+    tn = _net(3, 4, 8, 5, batches[0][0])
+    plan = PL.sweep_plan(tn, PL.grid_site_order(3, 4, open_last=[8]))
+    sliced = PL.choose_slices(tn, plan, n_sliced)[0]
+    p = compile_plan(tn, plan, sliced, group_bits=group_bits, precision=precision, bitstrings=batches[0])
+    for batch in batches + batches[:1]:
+        got = p.run(batch)
+        assert got.shape == (count, 2)
+        want = np.array([[_amp(sv, list(b.replace("x", v))) for v in "01"] for b in batch])
+        assert np.max(np.abs(got - want)) <= (1e-12 if precision == "uniform" else 1e-5) * np.max(np.abs(want))
+    p.close()
