@@ -102,6 +102,35 @@ __global__ void k_convert(const S* __restrict__ src, D* __restrict__ dst, int64_
   }
 }
 
+// Output columns of a bitstring batch: qubit q's leaf (grid x) gets column b
+// = [1, 0] or [0, 1] for its bit of bitstring b.  The words travel in the
+// kernel arguments, SET_BITS_WORDS per launch, so nothing is copied or
+// waited for; a batch was one copy and one synchronisation per qubit, and 64
+// bitstrings over 25 qubits then took 0.33 ms of a 1.69 ms run.
+struct OutCol {
+  void* ptr;     // the leaf's first element
+  int32_t bit;   // the qubit's bit in a bitstring word
+};
+#define SET_BITS_WORDS 256
+struct BitWords {
+  uint64_t w[SET_BITS_WORDS];
+};
+template <typename C>
+__global__ __launch_bounds__(SET_BITS_WORDS) void k_set_bits(const OutCol* __restrict__ cols, BitWords words,
+                                                             int64_t first, int n) {
+  const int t = (int)threadIdx.x;
+  if (t >= n) return;
+  const OutCol q = cols[blockIdx.x];
+  const bool one = (words.w[t] >> q.bit) & 1;
+  C v0, v1;
+  v0.x = one ? 0 : 1;
+  v1.x = one ? 1 : 0;
+  v0.y = v1.y = 0;
+  C* dst = reinterpret_cast<C*>(q.ptr) + 2 * (first + t);
+  dst[0] = v0;
+  dst[1] = v1;
+}
+
 size_t esize_of(int dtype) { return dtype == PQ_C128 ? 16 : 8; }
 
 struct Slot {
@@ -179,6 +208,7 @@ struct pq_plan {
     int slot, bit;                   // leaf slot of a closed output qubit, its bit in a bitstring word
   };
   std::vector<OutQubit> outq;        // a bitstring batch's closed output qubits (pq_plan_set_bitstrings)
+  OutCol* outq_dev = nullptr;        // ... and where their columns are, on the device
   int n_out_bits = 0;                // the top n_out_bits sliced bonds number output batches
   int64_t n_out = 1;                 // 2^n_out_bits results of out_elems each
   int out_slot = -1;
@@ -228,6 +258,7 @@ void free_plan(pq_ctx* c, pq_plan* p) {
   if (p->scratch) hipFree(p->scratch);
   if (p->out_dev) hipFree(p->out_dev);
   if (p->descs) hipFree(p->descs);
+  if (p->outq_dev) hipFree(p->outq_dev);
   if (p->chain_tab) hipFree(p->chain_tab);
   if (p->forest_buf) hipFree(p->forest_buf);
   for (auto& v : p->lev)
@@ -947,6 +978,19 @@ int create_plan(pq_ctx* c, const pq_plan_desc* d, int out_in_group, pq_plan** ou
     if (!is_contiguous(*t) || numel(*t) != ((int64_t)2 << d->n_out_bits))
       return bad("an output qubit's leaf must be a contiguous [2, 2^n_out_bits] tensor");
     p->outq.push_back({s, b});
+  }
+  if (!p->outq.empty()) {
+    std::vector<OutCol> cols;
+    for (const auto& q : p->outq) {
+      const Slot& sl = p->slots[q.slot];
+      cols.push_back({(unsigned char*)sl.leaf_buf->ptr + sl.leaf_off * (int64_t)c->esize, q.bit});
+    }
+    if (hipMalloc((void**)&p->outq_dev, cols.size() * sizeof(OutCol)) != hipSuccess ||
+        hipMemcpy(p->outq_dev, cols.data(), cols.size() * sizeof(OutCol), hipMemcpyHostToDevice) != hipSuccess) {
+      (void)hipGetLastError();
+      free_plan(c, p);
+      return fail(c, PQ_ERR_OOM, "output-qubit table upload failed");
+    }
   }
   // Steps.
   int64_t mpos = 0;
@@ -1746,23 +1790,18 @@ int pq_plan_set_bitstrings(pq_ctx* c, pq_plan* p, int n, const uint64_t* bits) {
   if (p->outq.empty()) return fail(c, PQ_ERR_ARG, "the plan has no bitstring batch");
   const int64_t nb = (int64_t)1 << p->n_out_bits;
   if (n < 1 || (int64_t)n > nb || !bits) return fail(c, PQ_ERR_ARG, "bitstring count out of range");
-  const size_t es = esize_of(c->dtype);
-  std::vector<unsigned char> col((size_t)(2 * nb) * es);
-  for (const auto& q : p->outq) {
-    std::fill(col.begin(), col.end(), 0);
-    for (int64_t b = 0; b < nb; ++b) {
-      const uint64_t w = bits[b < n ? b : 0];
-      const int64_t e = 2 * b + (int64_t)((w >> q.bit) & 1);   // column b: [1, 0] or [0, 1]
-      if (c->dtype == PQ_C128)
-        reinterpret_cast<double*>(col.data())[2 * e] = 1.0;
-      else
-        reinterpret_cast<float*>(col.data())[2 * e] = 1.0f;
-    }
-    const Slot& sl = p->slots[q.slot];
-    void* dst = (unsigned char*)sl.leaf_buf->ptr + sl.leaf_off * (int64_t)es;
-    hipError_t e = hipMemcpyAsync(dst, col.data(), col.size(), hipMemcpyHostToDevice, c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-    if (e != hipSuccess) return hipfail(c, e, "bitstring upload");
+  BitWords words;
+  for (int64_t first = 0; first < nb; first += SET_BITS_WORDS) {
+    const int m = (int)std::min<int64_t>(nb - first, SET_BITS_WORDS);
+    for (int t = 0; t < m; ++t) words.w[t] = bits[first + t < n ? first + t : 0];
+    if (c->dtype == PQ_C128)
+      hipLaunchKernelGGL((k_set_bits<c128>), dim3((unsigned)p->outq.size()), dim3(SET_BITS_WORDS), 0, c->stream,
+                         p->outq_dev, words, first, m);
+    else
+      hipLaunchKernelGGL((k_set_bits<c64>), dim3((unsigned)p->outq.size()), dim3(SET_BITS_WORDS), 0, c->stream,
+                         p->outq_dev, words, first, m);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return hipfail(c, e, "bitstring kernel");
   }
   return PQ_OK;
 }
