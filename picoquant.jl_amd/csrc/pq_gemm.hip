@@ -5,7 +5,7 @@
 //
 // m, n, k are linear indices of the M / N / K index groups; element offsets
 // come from per-workgroup offset tables in LDS (row tables for the tile,
-// K tables in windows of 2048), so any stride pattern is read and written
+// K tables in windows of 1024), so any stride pattern is read and written
 // in place.
 //
 // Complex product as four real MFMAs on split planes:
@@ -14,8 +14,8 @@
 // complex128 -> v_mfma_f64_16x16x4_f64 (fp64 accumulate)
 //
 // Tile: 256 lanes = 4 waves arranged WGM x WGN (2x2, 4x1 or 1x4); workgroup
-// tile BM x BN, each wave (BM/WGM) x (BN/WGN) as a grid of 16x16 MFMA tiles;
-// BK = 16 per LDS stage.  Extents below the tile are zero-padded.  Lane layout of a 16x16x4 MFMA (64 lanes): A operand lane l holds
+// tile BM x BN, each wave (BM/WGM) x (BN/WGN) as a grid of 16x16 MFMA tiles.
+// Extents below the tile are zero-padded.  Lane layout of a 16x16x4 MFMA (64 lanes): A operand lane l holds
 // A[l%16][l/16], B operand B[l/16][l%16]; accumulator register r holds
 // D[4*(l/16)+r][l%16] for f32 and D[l/16+4r][l%16] for f64.
 #include "pq_internal.h"
@@ -43,8 +43,7 @@ template <> struct mfma_t<double> {
   }
 };
 
-constexpr int BK = 16;
-constexpr int KTAB_MAX = 2048;   // K offsets held in LDS at a time
+constexpr int KTAB_MAX = 1024;   // K offsets that k_gemm holds in LDS at a time
 constexpr uint32_t GEMM_K_MAX = 1u << 24;
 
 // Workgroups are dealt to the 8 XCDs round-robin in launch order, and each
@@ -92,6 +91,45 @@ __device__ __forceinline__ void add_chunk(typename MF::acc (&accr)[TM][TN], type
       }
 }
 
+// One K step (4 values of K) of a wave's TM x TN complex blocks; fresh: the
+// sums start at zero.  Each real product runs over all blocks before the
+// next one, so consecutive MFMAs never wait for each other's accumulator.
+template <typename MF, int TM, int TN, typename C>
+__device__ __forceinline__ void mfma_step(typename MF::acc (&xr)[TM][TN], typename MF::acc (&xi)[TM][TN],
+                                          const C (&a)[TM], const C (&b)[TN], bool fresh) {
+  const typename MF::acc zero = {};
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) xr[i][j] = MF::op(a[i].x, b[j].x, fresh ? zero : xr[i][j]);
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) xi[i][j] = MF::op(a[i].x, b[j].y, fresh ? zero : xi[i][j]);
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) xr[i][j] = MF::op(-a[i].y, b[j].y, xr[i][j]);
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) xi[i][j] = MF::op(a[i].y, b[j].x, xi[i][j]);
+}
+
+// ------------------------------------------------------------------- k_gemm
+// Any stride pattern.  Element offsets are row offset + K offset: each
+// lane's row offsets stay in registers, the K offsets of a window of
+// KTAB_MAX indices in an LDS table.  The next K tile's elements are gathered
+// into registers while the matrix cores work on the current one, and LDS
+// holds interleaved complex values at an odd pitch, as in k_gemm2 (whose
+// main loop this is).
+// Bound: MFMA (79 % busy on a 2^13 x 2^9 x 2^11 complex64 product with every
+// index order shuffled; operands with unit stride along M and N take the same
+// time, so the gather is hidden).  That product: 738 us loading, storing and
+// multiplying each K tile in turn, 566 us with the register prefetch, 552 us
+// with each real product issued over all blocks; 2^11 x 2^7 x 2^9 complex128
+// 23.2 -> 16.8 us (calls overlapped on three streams).  K tiles of 32 take
+// the same time within 2 % and round more (longer first-level sums).
 template <typename C, int BM, int BN, int WGM, bool AK, bool BK_FAST>
 __global__ __launch_bounds__(256) void k_gemm(const C* __restrict__ A, const C* __restrict__ B,
                                               C* __restrict__ Out, GemmArgs g) {
@@ -100,12 +138,15 @@ __global__ __launch_bounds__(256) void k_gemm(const C* __restrict__ A, const C* 
   constexpr int WGN = 4 / WGM;
   constexpr int WM = BM / WGM, WN = BN / WGN;    // wave tile
   static_assert(WM % 16 == 0 && WN % 16 == 0, "wave tile must be a multiple of 16");
+  constexpr int BKT = 16;                        // K tile
   constexpr int TM = WM / 16, TN = WN / 16;      // 16x16 tiles per wave
   constexpr bool CHUNKED = sizeof(R) == 4;
+  constexpr int LDK = BKT + 1;                   // LDS row pitch (complex elements)
+  constexpr int ANE = BM * BKT / 256, BNE = BN * BKT / 256;   // elements per lane of each tile
 
-  __shared__ R As_r[BK][BM + 4], As_i[BK][BM + 4];
-  __shared__ R Bs_r[BK][BN + 4], Bs_i[BK][BN + 4];
-  __shared__ int32_t offAm[BM], offCm[BM], offBn[BN], offCn[BN];
+  __shared__ C As[BM * LDK], Bs[BN * LDK];
+  __shared__ int32_t offCm[BM], offCn[BN];
+  __shared__ int32_t offAm[BM], offBn[BN];
   __shared__ int32_t offAk[KTAB_MAX], offBk[KTAB_MAX];
 
   const uint32_t Mt = g.M.total, Nt = g.N.total, Kt = g.K.total;
@@ -121,18 +162,46 @@ __global__ __launch_bounds__(256) void k_gemm(const C* __restrict__ A, const C* 
     Out += oc;
   }
 
-  for (int t = tid; t < BM; t += 256) {
-    int32_t oa = 0, oc = 0;
-    if (m0 + t < Mt) group_offsets(g.M, m0 + t, oa, oc);
-    offAm[t] = oa;
-    offCm[t] = oc;
+  // rows past an operand's extent read its first row; their products only
+  // reach outputs that are never stored
+  for (int t = tid; t < BM + BN; t += 256) {
+    int32_t o = 0, oc = 0;
+    if (t < BM) {
+      if (m0 + t < Mt) group_offsets(g.M, m0 + t, o, oc);
+      offAm[t] = o;
+      offCm[t] = oc;
+    } else {
+      if (n0 + t - BM < Nt) group_offsets(g.N, n0 + t - BM, o, oc);
+      offBn[t - BM] = o;
+      offCn[t - BM] = oc;
+    }
   }
-  for (int t = tid; t < BN; t += 256) {
-    int32_t ob = 0, oc = 0;
-    if (n0 + t < Nt) group_offsets(g.N, n0 + t, ob, oc);
-    offBn[t] = ob;
-    offCn[t] = oc;
-  }
+  // K offsets of the window that starts at kb (entries past K: offset 0,
+  // zeroed when the tile is stored)
+  auto fill_window = [&](uint32_t kb) {
+    for (uint32_t t = tid; t < (uint32_t)KTAB_MAX && t < Kt - kb + BKT; t += 256) {
+      int32_t oa = 0, ob = 0;
+      if (kb + t < Kt) group_offsets(g.K, kb + t, oa, ob);
+      offAk[t] = oa;
+      offBk[t] = ob;
+    }
+  };
+  fill_window(0);
+  __syncthreads();
+
+  // This lane's elements of a tile: with the lanes along K, one K index and
+  // every 256 / BKT-th row; else every 256 / BM-th K index of one row
+  // (BM = 256 / BKT rows or more; a narrower tile's lanes wrap).
+  const int ak = AK ? tid % BKT : tid / BM, am = AK ? tid / BKT : tid % BM;
+  const int bk = BK_FAST ? tid % BKT : tid / BN, bn = BK_FAST ? tid / BKT : tid % BN;
+  constexpr int AKS = AK ? 0 : 256 / BM, AMS = AK ? 256 / BKT : 0;   // step per element
+  constexpr int BKS = BK_FAST ? 0 : 256 / BN, BNS = BK_FAST ? 256 / BKT : 0;
+  int32_t ga[AK ? ANE : 1], gb[BK_FAST ? BNE : 1];
+#pragma unroll
+  for (int q = 0; q < (AK ? ANE : 1); ++q) ga[q] = offAm[am + AMS * q];
+#pragma unroll
+  for (int q = 0; q < (BK_FAST ? BNE : 1); ++q) gb[q] = offBn[bn + BNS * q];
+
   const int wave = tid / 64, lane = tid % 64;
   const int wm = (wave / WGN) * WM, wn = (wave % WGN) * WN;
   const int li = lane % 16, lk = lane / 16;
@@ -140,71 +209,59 @@ __global__ __launch_bounds__(256) void k_gemm(const C* __restrict__ A, const C* 
   typename MF::acc accr[TM][TN], acci[TM][TN];
   zero_acc<MF, TM, TN>(accr, acci);
 
-  // K runs in windows of KTAB_MAX indices, each with its own offset table
-  // (every K tile of a window ends with a barrier, so the next window's
-  // table may overwrite the last one's)
-  for (uint32_t kb = 0; kb < Kt; kb += KTAB_MAX) {
-    const uint32_t ke = Kt - kb < (uint32_t)KTAB_MAX ? Kt : kb + KTAB_MAX;
-    for (uint32_t t = tid; t < ke - kb; t += 256) {
-      int32_t oa, ob;
-      group_offsets(g.K, kb + t, oa, ob);
-      offAk[t] = oa;
-      offBk[t] = ob;
+  C ra[ANE], rb[BNE];
+  auto load_tile = [&](uint32_t k0) {            // k0: the tile's place in the window
+#pragma unroll
+    for (int q = 0; q < ANE; ++q) ra[q] = A[ga[AK ? q : 0] + offAk[k0 + ak + AKS * q]];
+#pragma unroll
+    for (int q = 0; q < BNE; ++q) rb[q] = B[gb[BK_FAST ? q : 0] + offBk[k0 + bk + BKS * q]];
+  };
+  auto store_tile = [&](uint32_t left) {         // left: K values from this tile on
+    if (left < (uint32_t)BKT) {
+#pragma unroll
+      for (int q = 0; q < ANE; ++q)
+        if ((uint32_t)(ak + AKS * q) >= left) ra[q].x = ra[q].y = 0;
+#pragma unroll
+      for (int q = 0; q < BNE; ++q)
+        if ((uint32_t)(bk + BKS * q) >= left) rb[q].x = rb[q].y = 0;
     }
-    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < ANE; ++q) As[(am + AMS * q) * LDK + ak + AKS * q] = ra[q];
+#pragma unroll
+    for (int q = 0; q < BNE; ++q) Bs[(bn + BNS * q) * LDK + bk + BKS * q] = rb[q];
+  };
 
-    for (uint32_t k0 = kb; k0 < ke; k0 += BK) {
-      typename MF::acc cr[TM][TN], ci[TM][TN];
-      if constexpr (CHUNKED) zero_acc<MF, TM, TN>(cr, ci);
-      // A tile BM x BK -> As[k][m]
-      for (int t = tid; t < BM * BK; t += 256) {
-        int m, k;
-        if (AK) { k = t % BK; m = t / BK; } else { m = t % BM; k = t / BM; }
-        C v;
-        v.x = 0; v.y = 0;
-        if (m0 + m < Mt && k0 + k < ke) v = A[offAm[m] + offAk[k0 - kb + k]];
-        As_r[k][m] = v.x;
-        As_i[k][m] = v.y;
+  const C* Ap = As + (wm + li) * LDK + lk;
+  const C* Bp = Bs + (wn + li) * LDK + lk;
+  load_tile(0);
+  for (uint32_t k0 = 0; k0 < Kt; k0 += BKT) {
+    typename MF::acc cr[TM][TN], ci[TM][TN];
+    store_tile(Kt - k0);
+    __syncthreads();
+    if (k0 + BKT < Kt) {
+      const uint32_t next = (k0 + BKT) % KTAB_MAX;
+      if (next == 0) {
+        // past the barrier every lane has read its offsets of this window
+        fill_window(k0 + BKT);
+        __syncthreads();
       }
-      // B tile BK x BN -> Bs[k][n]
-      for (int t = tid; t < BK * BN; t += 256) {
-        int n, k;
-        if (BK_FAST) { k = t % BK; n = t / BK; } else { n = t % BN; k = t / BN; }
-        C v;
-        v.x = 0; v.y = 0;
-        if (n0 + n < Nt && k0 + k < ke) v = B[offBk[k0 - kb + k] + offBn[n]];
-        Bs_r[k][n] = v.x;
-        Bs_i[k][n] = v.y;
-      }
-      __syncthreads();
-#pragma unroll
-      for (int kk = 0; kk < BK; kk += 4) {
-        R ar[TM], ai[TM], br[TN], bi[TN];
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          ar[i] = As_r[kk + lk][wm + 16 * i + li];
-          ai[i] = As_i[kk + lk][wm + 16 * i + li];
-        }
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          br[j] = Bs_r[kk + lk][wn + 16 * j + li];
-          bi[j] = Bs_i[kk + lk][wn + 16 * j + li];
-        }
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j) {
-            typename MF::acc& xr = CHUNKED ? cr[i][j] : accr[i][j];
-            typename MF::acc& xi = CHUNKED ? ci[i][j] : acci[i][j];
-            xr = MF::op(ar[i], br[j], xr);
-            xr = MF::op(-ai[i], bi[j], xr);
-            xi = MF::op(ar[i], bi[j], xi);
-            xi = MF::op(ai[i], br[j], xi);
-          }
-      }
-      if constexpr (CHUNKED) add_chunk<MF, TM, TN>(accr, acci, cr, ci);
-      __syncthreads();
+      load_tile(next);
     }
+#pragma unroll
+    for (int kk = 0; kk < BKT; kk += 4) {
+      C a[TM], b[TN];
+#pragma unroll
+      for (int i = 0; i < TM; ++i) a[i] = Ap[16 * i * LDK + kk];
+#pragma unroll
+      for (int j = 0; j < TN; ++j) b[j] = Bp[16 * j * LDK + kk];
+      // a K tile's first products start the tile's fresh sums
+      if constexpr (CHUNKED)
+        mfma_step<MF, TM, TN>(cr, ci, a, b, kk == 0);
+      else
+        mfma_step<MF, TM, TN>(accr, acci, a, b, false);
+    }
+    if constexpr (CHUNKED) add_chunk<MF, TM, TN>(accr, acci, cr, ci);
+    __syncthreads();
   }
 
   // Epilogue: accumulator register r of tile (i, j) holds D[MF::row(lk, r)][li].
@@ -366,7 +423,6 @@ __global__ __launch_bounds__(256) void k_gemm2(const C* __restrict__ A, const C*
 
   const C* Ap = As + (wm + li) * LDK + lk;
   const C* Bp = Bs + (wn + li) * LDK + lk;
-  const typename MF::acc zero = {};
   load_tile(0);
   for (uint32_t kt = 0; kt < ntiles; ++kt) {
     typename MF::acc cr[TM][TN], ci[TM][TN];
@@ -380,19 +436,11 @@ __global__ __launch_bounds__(256) void k_gemm2(const C* __restrict__ A, const C*
       for (int i = 0; i < TM; ++i) a[i] = Ap[16 * i * LDK + kk];
 #pragma unroll
       for (int j = 0; j < TN; ++j) b[j] = Bp[16 * j * LDK + kk];
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          typename MF::acc& xr = CHUNKED ? cr[i][j] : accr[i][j];
-          typename MF::acc& xi = CHUNKED ? ci[i][j] : acci[i][j];
-          // a K tile's first products start the tile's fresh sums
-          const bool fresh = CHUNKED && kk == 0;
-          xr = MF::op(a[i].x, b[j].x, fresh ? zero : xr);
-          xr = MF::op(-a[i].y, b[j].y, xr);
-          xi = MF::op(a[i].x, b[j].y, fresh ? zero : xi);
-          xi = MF::op(a[i].y, b[j].x, xi);
-        }
+      // a K tile's first products start the tile's fresh sums
+      if constexpr (CHUNKED)
+        mfma_step<MF, TM, TN>(cr, ci, a, b, kk == 0);
+      else
+        mfma_step<MF, TM, TN>(accr, acci, a, b, false);
     }
     if constexpr (CHUNKED) add_chunk<MF, TM, TN>(accr, acci, cr, ci);
     __syncthreads();

@@ -36,8 +36,8 @@ struct CopyArgs {
 struct GemmArgs {
   Group M, N, K;      // as GenArgs
   Batch L;            // batch entries on grid z
-  int32_t a_kfast;    // A's unit-stride mode is in K: lanes walk k when loading
-  int32_t b_kfast;    // B's unit-stride mode is in K
+  int32_t a_kfast;    // K's first mode has unit stride in A: lanes walk k when loading
+  int32_t b_kfast;    // ... in B
   int32_t tile;       // see pq_set_gemm_tile
   int32_t contig;     // first K mode unit-stride in A and B, 16-byte aligned runs
 };
