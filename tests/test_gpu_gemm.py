@@ -237,3 +237,45 @@ def test_gemm16_arithmetic_setting_and_fallback():
             ctx.set_arithmetic(2)
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("K", [4, 15, 17, 31, 33, 1023, 1024, 1025, 1057, 2049])
+def test_any_stride_kernel_k_remainders(ctx, K):
+    """The any-stride kernel (no K mode with unit stride in both operands) at
+    K values around its K tiles (16, 32) and its 1024-entry offset window,
+    free extents one past a tile, every tile that the automatic choice can
+    take; and K first in one operand only."""
+    rng = np.random.default_rng(K)
+    M, N = 65, 33
+    for a_kfast, b_kfast in ((False, False), (True, False), (False, True)):
+        A = rand(rng, (K, M)) if a_kfast else rand(rng, (M, K))
+        ia = [1, -1] if a_kfast else [-1, 1]
+        B = rand(rng, (K, N)) if b_kfast else rand(rng, (N, K))
+        ib = [1, -2] if b_kfast else [-2, 1]
+        for tile in (-1, 0, 3, 6, 9):
+            check(ctx, A, ia, B, ib, gemm(ctx, A, ia, B, ib, tile))
+
+
+@pytest.mark.parametrize("dims", [(7, 3, 5, 6, 11, 9), (37, 13, 9, 27, 21, 5), (3, 2, 40, 8, 4, 30)])
+def test_summed_modes_in_either_order(ctx, dims):
+    """Two summed modes whose unit-stride one is the first of neither operand,
+    of A, of B, or of both in turn (the launch puts it first)."""
+    a1, k1, a2, k2, b1, b2 = dims
+    rng = np.random.default_rng(sum(dims))
+    ext = {1: k1, 2: k2, -1: a1, -2: a2, -3: b1, -4: b2}
+    for ia, ib in (([-1, 1, -2, 2], [2, -3, 1, -4]), ([2, -1, 1, -2], [-3, 1, 2, -4]), ([-1, 2, 1, -2], [1, 2, -3, -4]),
+                   ([1, -1, -2, 2], [2, -3, -4, 1]), ([-1, -2, 1, 2], [-3, 2, 1, -4])):
+        A, B = rand(rng, [ext[x] for x in ia]), rand(rng, [ext[x] for x in ib])
+        check(ctx, A, ia, B, ib, gemm(ctx, A, ia, B, ib))
+
+
+@pytest.mark.parametrize("M,N", [(17, 17), (40, 48), (64, 130), (300, 20), (16, 400), (700, 300), (33, 2100)])
+def test_automatic_tile_choice(ctx, M, N):
+    """Few workgroups (the smaller tiles of each width class) and many, with
+    and without a split K, through the automatic choice."""
+    rng = np.random.default_rng(M * N)
+    for K in (24, 64, 3072):
+        if M * N * K > 2 ** 26:
+            continue
+        A, B = rand(rng, (K, M)), rand(rng, (K, N))
+        check(ctx, A, [1, -1], B, [1, -2], gemm(ctx, A, [1, -1], B, [1, -2]))
