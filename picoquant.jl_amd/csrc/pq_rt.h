@@ -85,6 +85,7 @@ struct pq_ctx {
   void* scratch = nullptr;  // split-K partials for eager calls
   size_t scratch_bytes = 0;
   void* blas = nullptr;     // rocBLAS handle on this stream (rocSOLVER SVD), created on first use
+  int32_t* pinned = nullptr;  // two words that small SVDs write for the host, created on first use
   void* noalloc_scratch = nullptr;  // this device's scratch array of pq_contract_noalloc
   // Extra streams for concurrent branches of a planned run (default priority,
   // created on first use); stream 0 of a plan's schedule is `stream`.

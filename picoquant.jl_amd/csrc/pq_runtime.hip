@@ -618,6 +618,7 @@ int pq_ctx_destroy(pq_ctx* c) {
   for (auto& kv : c->free_blocks) hipFree(kv.second);
   c->free_blocks.clear();
   if (c->scratch) hipFree(c->scratch);
+  if (c->pinned) hipHostFree(c->pinned);
   for (hipStream_t& a : c->aux)
     if (a) {
       hipStreamSynchronize(a);

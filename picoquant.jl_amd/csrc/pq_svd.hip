@@ -1,12 +1,14 @@
 // decompose_tensor on the GPU: the SVD split of one tensor into two
 // (src/backends/interactive.jl:130-152 -> src/layer1.jl:146-190), used by
 // compress_bond! / contract_mps_tensor_network_circuit! (src/layer2.jl:
-// 423-703).  The tensor is permuted to (left, right) and materialised as an
-// m x n column-major matrix, factorised by rocSOLVER's gesdd (economy U and
+// 423-703).  A matrix of at most 64 on its shorter side is split by the
+// library's own kernels (pq_jacobi.hip); a larger one is permuted to (left,
+// right) and materialised as an m x n column-major matrix, factorised by rocSOLVER's gesdd (economy U and
 // V^H), the bond dimension chi is taken from the normalised spectrum exactly
 // as the reference does, and one kernel writes B = U[:, :chi] sqrt(S) and
 // C = sqrt(S) V^H[:chi, :] as new context tensors.
 #include "pq_rt.h"
+#include "pq_jacobi.h"
 
 #include <rocblas/rocblas.h>
 #include <rocsolver/rocsolver.h>
@@ -143,6 +145,79 @@ int decompose_typed(pq_ctx* c, const Tensor& A, int64_t m, int64_t n, double thr
   return PQ_OK;
 }
 
+// The same split for a matrix that fits one workgroup (pq_jacobi.hip), read
+// through the tensor's strides.  done = false: not applicable or not
+// converged, nothing is returned and the library takes it.
+int decompose_small(pq_ctx* c, const Tensor& v, int nleft, int64_t m, int64_t n, double threshold, int max_rank,
+                    Buf*& Bb, Buf*& Cb, int& chi, bool& done) {
+  done = false;
+  const size_t es = c->esize;
+  if (!jacobi_fits(m, n, es)) return PQ_OK;
+  JacArgs j;
+  std::vector<Mode> left, right;
+  for (int q = 0; q < v.rank; ++q) (q < nleft ? left : right).push_back({v.dims[q], v.strides[q], 0});
+  if (!fill_group(j.gm, merge_modes(left)) || !fill_group(j.gn, merge_modes(right))) return PQ_OK;
+  if (!c->pinned && hipHostMalloc((void**)&c->pinned, 2 * sizeof(int32_t), 0) != hipSuccess) {
+    (void)hipGetLastError();
+    c->pinned = nullptr;
+    return PQ_OK;
+  }
+  const int64_t p = std::max(m, n), k = std::min(m, n), cap = max_rank > 0 ? std::min<int64_t>(k, max_rank) : k;
+  Buf* Q = new_buf(c, (size_t)(p * k) * es);
+  Buf* log = new_buf(c, jacobi_log_bytes(k, es));
+  Buf* meta = new_buf(c, sizeof(JacMeta));
+  Buf* B = new_buf(c, (size_t)(m * cap) * es);
+  Buf* C = new_buf(c, (size_t)(cap * n) * es);
+  auto release = [&]() {
+    for (Buf* b : {Q, log, meta})
+      if (b) unref(c, b);
+  };
+  auto drop = [&]() {
+    release();
+    for (Buf* b : {B, C})
+      if (b) unref(c, b);
+  };
+  if (!Q || !log || !meta || !B || !C) {
+    drop();
+    return fail(c, PQ_ERR_OOM, "SVD workspace allocation failed");
+  }
+  j.X = (const unsigned char*)v.buf->ptr + v.off * es;
+  j.m = (int32_t)m;
+  j.n = (int32_t)n;
+  j.Q = Q->ptr;
+  j.log = log->ptr;
+  j.meta = static_cast<JacMeta*>(meta->ptr);
+  j.B = B->ptr;
+  j.C = C->ptr;
+  // src/layer1.jl:166-175: threshold at least sqrt(eps), relative to the
+  // spectrum's 2-norm; max_rank caps the count
+  const double eps = c->dtype == PQ_C128 ? (double)std::numeric_limits<double>::epsilon()
+                                         : (double)std::numeric_limits<float>::epsilon();
+  j.thr = std::max(threshold, std::sqrt(eps));
+  j.max_rank = max_rank;
+  j.host = c->pinned;
+  hipError_t e = c->dtype == PQ_C128 ? launch_jacobi<c128>(j, c->stream) : launch_jacobi<c64>(j, c->stream);
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  if (e != hipSuccess) {
+    drop();
+    return hipfail(c, e, "small SVD");
+  }
+  if (c->pinned[1]) {
+    drop();
+    return PQ_OK;
+  }
+  done = true;
+  chi = c->pinned[0];
+  if (chi < 1) {
+    drop();
+    return fail(c, PQ_ERR_UNSUPPORTED, "decompose of a zero tensor (no singular value above the threshold)");
+  }
+  release();
+  Bb = B;
+  Cb = C;
+  return PQ_OK;
+}
+
 }  // namespace
 
 namespace pqrt {
@@ -181,15 +256,20 @@ int pq_decompose(pq_ctx* c, pq_tensor h, int nleft, const int32_t* left, int nri
     (q < nleft ? m : n) *= v.dims[q];
   }
   if (m < 1 || n < 1 || m > INT32_MAX || n > INT32_MAX) return fail(c, PQ_ERR_UNSUPPORTED, "matrix size out of range");
-  Tensor A;
-  int r = materialize_into(c, v, A);   // a private copy: gesdd overwrites it
-  if (r) return r;
   Buf *Bb = nullptr, *Cb = nullptr;
   int chi = 0;
-  r = c->dtype == PQ_C128 ? decompose_typed<c128, double>(c, A, m, n, threshold, max_rank, Bb, Cb, chi)
-                          : decompose_typed<c64, float>(c, A, m, n, threshold, max_rank, Bb, Cb, chi);
-  unref(c, A.buf);
+  bool done = false;
+  int r = decompose_small(c, v, nleft, m, n, threshold, max_rank, Bb, Cb, chi, done);
   if (r) return r;
+  if (!done) {
+    Tensor A;
+    r = materialize_into(c, v, A);   // a private copy: gesdd overwrites it
+    if (r) return r;
+    r = c->dtype == PQ_C128 ? decompose_typed<c128, double>(c, A, m, n, threshold, max_rank, Bb, Cb, chi)
+                            : decompose_typed<c64, float>(c, A, m, n, threshold, max_rank, Bb, Cb, chi);
+    unref(c, A.buf);
+    if (r) return r;
+  }
   Tensor B, Cn;
   B.buf = Bb;
   B.rank = nleft + 1;

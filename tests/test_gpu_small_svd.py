@@ -1,0 +1,122 @@
+"""pq_decompose on the one-workgroup SVD (shorter side at most 64) against
+numpy's SVD in complex128: the bond dimension, the split's product (the
+truncated matrix), the factors' norms (sqrt of the singular values) and
+orthogonality, over padded sizes (4, 8, 16, 32, 64 columns; 16 to 256 rows)
+and their edges, tall and wide, graded and rank-deficient spectra, strided
+tensors.
+
+Tolerance: a column passes at most about 10 sweeps x 63 rotations, each
+rounding at most 4 eps of the matrix norm: 2.8e-13 for complex128, 1.5e-4
+for complex64 (both relative to the largest singular value)."""
+import numpy as np
+import pytest
+
+from picoquant_hip import _lib
+
+pytestmark = pytest.mark.gpu
+
+TOL = {np.complex128: 2.8e-13, np.complex64: 1.5e-4}
+
+
+@pytest.fixture(scope="module", params=[np.complex128, np.complex64], ids=["c128", "c64"])
+def ctx(request):
+    c = _lib.Context(request.param)
+    yield c
+    c.close()
+
+
+def rnd(rng, m, n):
+    return rng.standard_normal((m, n)) + 1j * rng.standard_normal((m, n))
+
+
+def graded(rng, m, n, digits):
+    k = min(m, n)
+    u, w = np.linalg.qr(rnd(rng, m, k))[0], np.linalg.qr(rnd(rng, n, k))[0]
+    return (u * np.logspace(0, -digits, k)) @ w.conj().T
+
+
+def check(ctx, A, B, C, chi, threshold=0.0, max_rank=0):
+    tol = TOL[ctx.np_dtype.type]
+    u, s, vh = np.linalg.svd(A)
+    thr = max(threshold, np.sqrt(np.finfo(ctx.np_dtype).eps))
+    rel = s / np.linalg.norm(s)
+    want = int(np.sum(rel > thr))
+    sure = int(np.sum(rel > thr + 4 * tol))          # values at the cut-off may fall either way
+    maybe = int(np.sum(rel > thr - 4 * tol))
+    if max_rank > 0:
+        want, sure, maybe = (min(x, max_rank) for x in (want, sure, maybe))
+    assert sure <= chi <= maybe, (chi, want)
+    assert B.shape == (A.shape[0], chi) and C.shape == (chi, A.shape[1])
+    trunc = (u[:, :chi] * s[:chi]) @ vh[:chi]
+    gap = s[chi - 1] - s[chi] if chi < len(s) else s[chi - 1]
+    # a truncated product is defined up to tol x norm / gap
+    assert np.linalg.norm(B @ C - trunc) <= tol * s[0] * max(1.0, s[0] / max(gap, 1e-300) if chi < len(s) else 1.0)
+    assert np.all(np.abs(np.sum(np.abs(B) ** 2, axis=0) - s[:chi]) <= tol * s[0])
+    assert np.all(np.abs(np.sum(np.abs(C) ** 2, axis=1) - s[:chi]) <= tol * s[0])
+    for g in (B.conj().T @ B, C @ C.conj().T):
+        assert np.max(np.abs(g - np.diag(s[:chi]))) <= tol * s[0]
+
+
+def split(ctx, A, threshold=0.0, max_rank=0):
+    h = ctx.upload(A.astype(ctx.np_dtype))
+    hb, hc, chi = ctx.decompose(h, [1], [2], threshold, max_rank)
+    B, C = ctx.download(hb), ctx.download(hc)
+    for x in (h, hb, hc):
+        ctx.free(x)
+    return B.astype(np.complex128), C.astype(np.complex128), chi
+
+
+SHAPES = [(1, 1), (1, 7), (9, 1), (2, 2), (4, 4), (5, 4), (4, 16), (8, 8), (9, 8), (16, 16), (17, 16), (8, 32),
+          (32, 8), (31, 33), (32, 32), (65, 32), (128, 16), (129, 16), (256, 4), (3, 256), (257, 4), (48, 48), (64, 33),
+          (64, 64), (63, 64), (65, 64), (70, 66)]
+
+
+@pytest.mark.parametrize("m,n", SHAPES)
+def test_shapes(ctx, m, n):
+    A = rnd(np.random.default_rng(1000 * m + n), m, n).astype(ctx.np_dtype).astype(np.complex128)
+    check(ctx, A, *split(ctx, A))
+    if min(m, n) > 2:
+        r = min(m, n) // 2
+        check(ctx, A, *split(ctx, A, max_rank=r), max_rank=r)
+
+
+@pytest.mark.parametrize("m,n", [(4, 4), (8, 6), (24, 16), (20, 32), (64, 64), (100, 20)])
+@pytest.mark.parametrize("digits", [3, 12, 20])
+def test_graded_spectra(ctx, m, n, digits):
+    """Singular values falling over `digits` decades, far below the cut-off."""
+    A = graded(np.random.default_rng(m + n + digits), m, n, digits).astype(ctx.np_dtype).astype(np.complex128)
+    check(ctx, A, *split(ctx, A))
+    check(ctx, A, *split(ctx, A, threshold=1e-2), threshold=1e-2)
+
+
+def test_rank_deficient_degenerate_and_scaled(ctx):
+    rng = np.random.default_rng(5)
+    low = rnd(rng, 40, 6) @ rnd(rng, 6, 30)
+    unit = np.linalg.qr(rnd(rng, 32, 32))[0]            # every singular value 1
+    sparse = np.zeros((16, 16), complex)
+    sparse[3, 5], sparse[7, 5], sparse[3, 11] = 2, 1j, -1
+    for A in (low, unit, sparse, np.eye(64), 1e-30 * rnd(rng, 12, 20), 1e30 * rnd(rng, 64, 40)):
+        A = A.astype(ctx.np_dtype).astype(np.complex128)
+        check(ctx, A, *split(ctx, A))
+    with pytest.raises(_lib.PQError) as e:
+        split(ctx, np.zeros((16, 8)))
+    assert e.value.code == _lib.PQ_ERR_UNSUPPORTED
+
+
+def test_strided_tensor(ctx):
+    """A permuted, sliced rank-5 tensor split across its axes."""
+    rng = np.random.default_rng(6)
+    T = (rng.standard_normal((3, 4, 2, 5, 4)) + 1j * rng.standard_normal((3, 4, 2, 5, 4)))
+    T = T.astype(ctx.np_dtype).astype(np.complex128)
+    h = ctx.upload(T.astype(ctx.np_dtype))
+    hp = ctx.permute(h, [4, 1, 5, 3, 2])
+    hv = ctx.view(hp, 1, 2, 4)
+    ref = np.transpose(T, (3, 0, 4, 2, 1))[1:4]
+    hb, hc, chi = ctx.decompose(hv, [2, 5], [4, 1, 3])
+    B, C = ctx.download(hb), ctx.download(hc)
+    assert B.shape == (3, 4, chi) and C.shape == (chi, 2, 3, 4)
+    A = np.transpose(ref, (1, 4, 3, 0, 2)).reshape(12, 24, order="F")
+    check(ctx, A, B.reshape(12, chi, order="F"), C.reshape(chi, 24, order="F"), chi)
+    assert np.array_equal(ctx.download(h), T.astype(ctx.np_dtype))       # not consumed
+    for x in (h, hp, hv, hb, hc):
+        ctx.free(x)
