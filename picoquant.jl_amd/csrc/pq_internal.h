@@ -30,6 +30,20 @@ struct CopyArgs {
   Group G;
 };
 
+// Strided copy through LDS tiles of 2^CB_BITS elements: `nb` bits (extent-2
+// factors of the copy's modes) make a tile, the other factors (`outer`: s0 =
+// input stride, s1 = output stride) number the tiles.  Bit i of a lane's
+// load index has input stride is[i] and LDS address vector il[i], bit i of
+// its store index output stride os[i] and LDS address vector ol[i]; strides
+// add, LDS vectors XOR.
+#define CB_BITS(es) ((es) == 16 ? 11 : 12)
+#define CB_MAX 12
+struct CopyBitsArgs {
+  Group outer;
+  int32_t is[CB_MAX], os[CB_MAX];
+  int32_t il[CB_MAX], ol[CB_MAX];
+};
+
 // Tiled GEMM on MFMA with gathered operand loads and scattered C stores.
 // Offsets are split as (row group, col group) so a tile loads through two
 // small tables instead of per-element decoding.
@@ -111,6 +125,8 @@ hipError_t launch_reduce(const C* A, const C* B, C* Out, const GenArgs& a, C* pa
                          int nblocks, hipStream_t s);
 template <typename C>
 hipError_t launch_copy(const C* In, C* Out, const CopyArgs& a, hipStream_t s);
+template <typename C>
+hipError_t launch_copy_bits(const C* In, C* Out, const CopyBitsArgs& a, hipStream_t s);
 template <typename C>
 hipError_t launch_gemm(const C* A, const C* B, C* Out, const GemmArgs& a, hipStream_t s);
 // Split-K second pass: Out[C offset of (m, n)] = sum over z < parts of

@@ -211,6 +211,62 @@ __global__ __launch_bounds__(256) void k_copy(const C* __restrict__ In, C* __res
   }
 }
 
+// ------------------------------------------------------------- k_copy_bits
+// One tile per workgroup: loaded along its input runs, put into LDS, stored
+// along its output runs.  The offsets are sums over index bits, a lane's
+// low 8 bits once, the rest uniform, where k_copy decodes every element
+// through all modes and reads one element of each line it touches.
+// Bound: HBM (2^24 complex64 elements in a random axis order: 48 us = 5.5
+// TB/s, 107 us by k_copy, whose time is its per-element decode).
+template <typename C>
+__global__ __launch_bounds__(256) void k_copy_bits(const C* __restrict__ In, C* __restrict__ Out, CopyBitsArgs a) {
+  constexpr int NB = CB_BITS(sizeof(C)), PER = 1 << (NB - 8);
+  __shared__ C tile[1 << NB];
+  int32_t bi, bo;
+  group_offsets(a.outer, blockIdx.x, bi, bo);
+  const int tid = threadIdx.x;
+  int32_t li = 0, lo = 0, ai = 0, ao = 0;
+#pragma unroll
+  for (int b = 0; b < 8; ++b) {
+    const int32_t m = -((tid >> b) & 1);
+    li += m & a.is[b];
+    lo += m & a.os[b];
+    ai ^= m & a.il[b];
+    ao ^= m & a.ol[b];
+  }
+  const C* in = In + bi;
+  C* out = Out + bo;
+  C v[PER];
+#pragma unroll
+  for (int q = 0; q < PER; ++q) {
+    int32_t o = li;
+#pragma unroll
+    for (int b = 8; b < NB; ++b)
+      if ((q >> (b - 8)) & 1) o += a.is[b];
+    v[q] = in[o];
+  }
+#pragma unroll
+  for (int q = 0; q < PER; ++q) {
+    int32_t t = ai;
+#pragma unroll
+    for (int b = 8; b < NB; ++b)
+      if ((q >> (b - 8)) & 1) t ^= a.il[b];
+    tile[t] = v[q];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < PER; ++q) {
+    int32_t o = lo, t = ao;
+#pragma unroll
+    for (int b = 8; b < NB; ++b)
+      if ((q >> (b - 8)) & 1) {
+        o += a.os[b];
+        t ^= a.ol[b];
+      }
+    out[o] = tile[t];
+  }
+}
+
 // ----------------------------------------------------------------- k_multi
 // Grouped small contractions: problem blockIdx.y, batch entry blockIdx.z,
 // one lane per output element (grid-stride over blockIdx.x), loop over K;
@@ -474,6 +530,12 @@ hipError_t launch_copy(const C* In, C* Out, const CopyArgs& a, hipStream_t s) {
 }
 
 template <typename C>
+hipError_t launch_copy_bits(const C* In, C* Out, const CopyBitsArgs& a, hipStream_t s) {
+  hipLaunchKernelGGL((k_copy_bits<C>), dim3(a.outer.total), dim3(256), 0, s, In, Out, a);
+  return hipGetLastError();
+}
+
+template <typename C>
 hipError_t launch_multi(const MultiDesc* descs, int n, unsigned blocks_x, unsigned batch, int64_t group,
                         hipStream_t s) {
   if (n < 1 || n > 65535 || batch < 1 || batch > 65535) return hipErrorInvalidValue;
@@ -496,6 +558,7 @@ hipError_t launch_forest(const ForestStep* steps, const int4* items, const int2*
   template hipError_t launch_stream<C>(const C*, const C*, C*, const StreamArgs&, hipStream_t);      \
   template hipError_t launch_generic<C>(const C*, const C*, C*, const GenArgs&, hipStream_t);        \
   template hipError_t launch_reduce<C>(const C*, const C*, C*, const GenArgs&, C*, int, hipStream_t); \
-  template hipError_t launch_copy<C>(const C*, C*, const CopyArgs&, hipStream_t);
+  template hipError_t launch_copy<C>(const C*, C*, const CopyArgs&, hipStream_t);                    \
+  template hipError_t launch_copy_bits<C>(const C*, C*, const CopyBitsArgs&, hipStream_t);
 PQ_INST(c128)
 PQ_INST(c64)

@@ -186,6 +186,81 @@ static C* dptr(const Tensor& t) {
   return reinterpret_cast<C*>(t.buf->ptr) + t.off;
 }
 
+// Splits a copy (modes in output order, s0 = input stride, s1 = output
+// stride) into an LDS tile's bits and its outer modes.  The tile holds the
+// six factors of two with the smallest input strides and the six with the
+// smallest output strides, so both sides move runs of 512 bytes or more
+// where the tensor has them, and the next output bits up to its size.  Not
+// for copies whose runs are long already (32 elements or more lie the same
+// way on both sides), small ones (below 2^15 elements the launch is the
+// cost), or where fewer factors of two exist than a tile has bits (odd
+// extents): k_copy takes those.
+static bool copy_bits_args(const std::vector<Mode>& modes, size_t esize, CopyBitsArgs& a) {
+  const int nb = CB_BITS(esize);
+  int64_t total = 1;
+  for (const Mode& m : modes) total *= m.ext;
+  if (total < (1 << 15) || modes.empty() || (modes[0].s0 == 1 && modes[0].ext >= 32)) return false;
+  struct Bit {
+    int64_t in, out;
+    int mode, tile;
+  };
+  std::vector<Bit> bits;
+  for (size_t q = 0; q < modes.size(); ++q)
+    for (int k = 0; ((modes[q].ext >> k) & 1) == 0; ++k)
+      bits.push_back({modes[q].s0 << k, modes[q].s1 << k, (int)q, -1});
+  if ((int)bits.size() < nb) return false;
+  std::vector<int> by_in(bits.size()), by_out(bits.size());
+  for (size_t i = 0; i < bits.size(); ++i) by_in[i] = by_out[i] = (int)i;
+  std::stable_sort(by_in.begin(), by_in.end(), [&](int x, int y) { return bits[x].in < bits[y].in; });
+  std::stable_sort(by_out.begin(), by_out.end(), [&](int x, int y) { return bits[x].out < bits[y].out; });
+  // a mode's bits enter its tile part from its fastest on, so that the rest
+  // of the mode is one outer mode
+  std::vector<int> taken(modes.size(), 0);
+  int n = 0;
+  auto take = [&](int i) {
+    Bit& b = bits[i];
+    if (b.tile >= 0 || n == nb) return;
+    b.tile = n++;
+    ++taken[b.mode];
+  };
+  for (int k = 0; k < 6; ++k) take(by_in[k]);
+  for (int k = 0; k < 6; ++k) take(by_out[k]);
+  for (int i : by_out) take(i);
+  // load order: by input stride; store order: by output stride.  LDS: load
+  // bit i is address bit i; the store's low bits that are not among the
+  // load's low bits also flip an unused low address bit each, so the 64
+  // lanes of either access fall on distinct banks.
+  std::vector<int> li, lo;
+  for (int i : by_in)
+    if (bits[i].tile >= 0) li.push_back(i);
+  for (int i : by_out)
+    if (bits[i].tile >= 0) lo.push_back(i);
+  std::vector<int32_t> vec(bits.size(), 0);
+  for (int k = 0; k < nb; ++k) vec[li[k]] = 1 << k;
+  const int low = 6;
+  uint32_t used = 0;
+  for (int k = 0; k < low; ++k)
+    if (vec[lo[k]] < (1 << low)) used |= (uint32_t)vec[lo[k]];
+  for (int k = 0; k < low; ++k)
+    if (vec[lo[k]] >= (1 << low)) {
+      int f = 0;
+      while ((used >> f) & 1) ++f;
+      used |= 1u << f;
+      vec[lo[k]] |= 1 << f;
+    }
+  memset(&a, 0, sizeof(a));
+  for (int k = 0; k < nb; ++k) {
+    a.is[k] = (int32_t)bits[li[k]].in;
+    a.il[k] = vec[li[k]];
+    a.os[k] = (int32_t)bits[lo[k]].out;
+    a.ol[k] = vec[lo[k]];
+  }
+  std::vector<Mode> outer;
+  for (size_t q = 0; q < modes.size(); ++q)
+    outer.push_back({modes[q].ext >> taken[q], modes[q].s0 << taken[q], modes[q].s1 << taken[q]});
+  return fill_group(a.outer, merge_modes(outer));
+}
+
 int materialize_into(pq_ctx* c, const Tensor& src, Tensor& dst) {
   dst = Tensor();
   dst.rank = src.rank;
@@ -203,10 +278,16 @@ int materialize_into(pq_ctx* c, const Tensor& src, Tensor& dst) {
     unref(c, dst.buf);
     return fail(c, PQ_ERR_UNSUPPORTED, "tensor too large or too fragmented");
   }
+  CopyBitsArgs cb;
+  const bool tiled = copy_bits_args(modes, c->esize, cb);
   ProfScope ps(c, PQ_KC_COPY, 2.0 * n * c->esize, 0);
-  hipError_t e = (c->dtype == PQ_C128)
-                     ? launch_copy<c128>(dptr<c128>(src), dptr<c128>(dst), a, c->stream)
-                     : launch_copy<c64>(dptr<c64>(src), dptr<c64>(dst), a, c->stream);
+  hipError_t e;
+  if (c->dtype == PQ_C128)
+    e = tiled ? launch_copy_bits<c128>(dptr<c128>(src), dptr<c128>(dst), cb, c->stream)
+              : launch_copy<c128>(dptr<c128>(src), dptr<c128>(dst), a, c->stream);
+  else
+    e = tiled ? launch_copy_bits<c64>(dptr<c64>(src), dptr<c64>(dst), cb, c->stream)
+              : launch_copy<c64>(dptr<c64>(src), dptr<c64>(dst), a, c->stream);
   if (e != hipSuccess) return hipfail(c, e, "copy kernel");
   return PQ_OK;
 }
