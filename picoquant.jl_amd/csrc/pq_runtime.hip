@@ -433,13 +433,14 @@ int resolve_step(pq_ctx* c, StepSpec& s, size_t esize) {
       s.tile = pick_tile(s, m, n, esize);
     s.splitk = kc == PQ_KC_GEMM ? gemm_split(s, s.tile, m, n) : 1;
     // The order of the summed modes is free.  One that runs with unit stride
-    // in an operand goes first, so that lanes along K read adjacent elements
+    // in an operand for 8 elements or more (a line of complex128) goes
+    // first, so that lanes along K read adjacent elements
     // (bond tensors with six extents of 48, complex64: 3.31 -> 0.94 ms; 1665
     // x 351 x 693 complex128: 73 -> 67 us); a split product keeps its
     // order, as it cuts the last mode.
     if (s.splitk == 1 && s.K.size() > 1 && s.K[0].s0 != 1 && s.K[0].s1 != 1)
       for (size_t q = 1; q < s.K.size(); ++q)
-        if (s.K[q].s0 == 1 || s.K[q].s1 == 1) {
+        if ((s.K[q].s0 == 1 || s.K[q].s1 == 1) && s.K[q].ext >= 8) {
           std::rotate(s.K.begin(), s.K.begin() + q, s.K.begin() + q + 1);
           break;
         }
