@@ -125,6 +125,10 @@ hipError_t launch_reduce(const C* A, const C* B, C* Out, const GenArgs& a, C* pa
                          int nblocks, hipStream_t s);
 template <typename C>
 hipError_t launch_copy(const C* In, C* Out, const CopyArgs& a, hipStream_t s);
+// Writes n 32-bit words of host data to device memory, the data in the
+// kernel's arguments (copied when the launch returns).
+#define PQ_PUT_WORDS 256
+hipError_t launch_put(void* dst, const void* host, int n, hipStream_t s);
 template <typename C>
 hipError_t launch_copy_bits(const C* In, C* Out, const CopyBitsArgs& a, hipStream_t s);
 template <typename C>

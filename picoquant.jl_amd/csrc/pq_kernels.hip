@@ -12,6 +12,7 @@
 //              (materialises permuted / sliced views).
 #include "pq_internal.h"
 
+#include <cstring>
 #include <type_traits>
 
 namespace {
@@ -209,6 +210,14 @@ __global__ __launch_bounds__(256) void k_copy(const C* __restrict__ In, C* __res
     group_offsets(a.G, t, oi, oo);
     Out[oo] = In[oi];
   }
+}
+
+// -------------------------------------------------------------------- k_put
+struct PutWords {
+  uint32_t w[PQ_PUT_WORDS];
+};
+__global__ __launch_bounds__(PQ_PUT_WORDS) void k_put(uint32_t* __restrict__ dst, PutWords a, int n) {
+  if ((int)threadIdx.x < n) dst[threadIdx.x] = a.w[threadIdx.x];
 }
 
 // ------------------------------------------------------------- k_copy_bits
@@ -526,6 +535,14 @@ hipError_t launch_reduce(const C* A, const C* B, C* Out, const GenArgs& a, C* pa
 template <typename C>
 hipError_t launch_copy(const C* In, C* Out, const CopyArgs& a, hipStream_t s) {
   hipLaunchKernelGGL((k_copy<C>), dim3(grid_for(a.G.total, 256)), dim3(256), 0, s, In, Out, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_put(void* dst, const void* host, int n, hipStream_t s) {
+  if (n < 1 || n > PQ_PUT_WORDS) return hipErrorInvalidValue;
+  PutWords a;
+  memcpy(a.w, host, (size_t)n * 4);
+  hipLaunchKernelGGL(k_put, dim3(1), dim3(n <= 64 ? 64 : PQ_PUT_WORDS), 0, s, (uint32_t*)dst, a, n);
   return hipGetLastError();
 }
 

@@ -731,9 +731,12 @@ int pq_synchronize(pq_ctx* c) {
 namespace {
 
 // Stream-ordered copy of n host elements (host_dtype) into device memory of
-// the context's element type, converting on the host when the types differ;
-// synchronises, so the host buffer may be reused on return.
-hipError_t host_to_device(pq_ctx* c, void* dst, const void* host, int host_dtype, int64_t n) {
+// the context's element type, converting on the host when the types differ.
+// The host buffer may be reused on return: synchronises, unless `wait` is
+// false and the data (a gate, an input vector: at most 1 KiB) fits a
+// kernel's arguments -- a copy with its synchronisation is 17 us of a
+// program that builds a network gate by gate, the launch 4.
+hipError_t host_to_device(pq_ctx* c, void* dst, const void* host, int host_dtype, int64_t n, bool wait) {
   if (n <= 0) return hipSuccess;
   std::vector<unsigned char> tmp;
   const void* src = host;
@@ -749,6 +752,10 @@ hipError_t host_to_device(pq_ctx* c, void* dst, const void* host, int host_dtype
       for (int64_t i = 0; i < 2 * n; ++i) d[i] = (double)s[i];
     }
     src = tmp.data();
+  }
+  if (!wait && n * (int64_t)c->esize <= 4 * PQ_PUT_WORDS) {
+    c->unsynced = true;
+    return launch_put(dst, src, (int)(n * (int64_t)c->esize / 4), c->stream);
   }
   hipError_t e = hipMemcpyAsync(dst, src, (size_t)n * c->esize, hipMemcpyHostToDevice, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
@@ -774,7 +781,7 @@ int pq_tensor_upload(pq_ctx* c, int rank, const int64_t* dims, const void* host,
   if (n > 0 && !host) return fail(c, PQ_ERR_ARG, "null host pointer");
   t.buf = new_buf(c, (size_t)n * c->esize);
   if (!t.buf) return fail(c, PQ_ERR_OOM, "device allocation failed");
-  hipError_t e = host_to_device(c, t.buf->ptr, host, host_dtype, n);
+  hipError_t e = host_to_device(c, t.buf->ptr, host, host_dtype, n, false);
   if (e != hipSuccess) {
     unref(c, t.buf);
     return hipfail(c, e, "upload");
@@ -791,7 +798,7 @@ int pq_tensor_write(pq_ctx* c, pq_tensor h, const void* host, int host_dtype) {
   if (!is_contiguous(*t)) return fail(c, PQ_ERR_ARG, "tensor_write needs a contiguous tensor");
   const int64_t n = numel(*t);
   if (n > 0 && !host) return fail(c, PQ_ERR_ARG, "null host pointer");
-  hipError_t e = host_to_device(c, (unsigned char*)t->buf->ptr + t->off * c->esize, host, host_dtype, n);
+  hipError_t e = host_to_device(c, (unsigned char*)t->buf->ptr + t->off * c->esize, host, host_dtype, n, true);
   if (e != hipSuccess) return hipfail(c, e, "tensor write");
   return PQ_OK;
 }
@@ -958,6 +965,12 @@ int pq_tensor_device_ptr(pq_ctx* c, pq_tensor h, void** base, int64_t* off, int6
   if (!c) return PQ_ERR_ARG;
   Tensor* t = get(c, h);
   if (!t) return fail(c, PQ_ERR_NOT_FOUND, "unknown tensor handle");
+  // the caller may read the memory from a stream of its own
+  if (c->unsynced) {
+    hipError_t e = hipStreamSynchronize(c->stream);
+    if (e != hipSuccess) return hipfail(c, e, "device pointer sync");
+    c->unsynced = false;
+  }
   if (base) *base = t->buf->ptr;
   if (off) *off = t->off;
   if (strides)
