@@ -532,6 +532,20 @@ hipError_t launch_tile(const C* A, const C* B, C* Out, const GemmArgs& g, hipStr
 // B lane l holds B[8(l/16)+i][l%16], accumulator r holds D[4(l/16)+r][l%16].
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+typedef float floatx2 __attribute__((ext_vector_type(2)));
+typedef uint32_t uint2v __attribute__((ext_vector_type(2)));
+
+// Two values rounded to fp16, in one word, and what the rounding left of
+// them (exact: x - fp16(x), the word's halves read in place).
+__device__ __forceinline__ uint32_t pack16(const floatx2& x) {
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(x, half2v));
+}
+__device__ __forceinline__ floatx2 rest16(uint32_t h, const floatx2& x) {
+  floatx2 r;
+  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(r.x) : "v"(h), "v"(x.x));
+  asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r.y) : "v"(h), "v"(x.y));
+  return r;
+}
 
 __device__ __forceinline__ floatx4 mfma16(const half8& a, const half8& b, const floatx4& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
@@ -545,7 +559,7 @@ __global__ __launch_bounds__(256) void k_gemm_h(const c64* __restrict__ A, const
   constexpr int WM = BM / WGM, WN = BN / WGN;
   constexpr int TM = WM / 16, TN = WN / 16;
   static_assert(WM % 16 == 0 && WN % 16 == 0, "wave tile must be a multiple of 16");
-  constexpr int CPR = BKT / 2;                    // 16-byte chunks (2 complex) per row
+  constexpr int CPR = BKT / 4;                    // 32-byte units (4 complex) per row
   constexpr int ACH = (BM * CPR + 255) / 256;
   constexpr int BCH = (BN * CPR + 255) / 256;
   constexpr int KT_MAX = 2048 / BKT;
@@ -594,25 +608,25 @@ __global__ __launch_bounds__(256) void k_gemm_h(const c64* __restrict__ A, const
   }
   __syncthreads();
 
-  // Lane chunks: 16 consecutive lanes hold the 16 chunks of one row, so a
-  // row's scale is a reduction over a 16-lane group.  Rows past the
-  // operand read its first row; lanes past the tile use the spare row.
+  // Lane units: 8 consecutive lanes hold the 8 units of one row, so a row's
+  // scale is a maximum over half a DPP row.  Rows past the operand read its
+  // first row; lanes past the tile use the spare row.
   int32_t ga[ACH], gb[BCH], la[ACH], lb[BCH], ra_row[ACH], rb_row[BCH];
 #pragma unroll
   for (int q = 0; q < ACH; ++q) {
     const int id = tid + 256 * q;
     const int row = id / CPR, cc = id % CPR;
-    ga[q] = (row < BM ? offAm[row] : 0) + cc * 2;
+    ga[q] = (row < BM ? offAm[row] : 0) + cc * 4;
     ra_row[q] = row < BM ? row : BM;
-    la[q] = ra_row[q] * PK + cc * 2;
+    la[q] = ra_row[q] * PK + cc * 4;
   }
 #pragma unroll
   for (int q = 0; q < BCH; ++q) {
     const int id = tid + 256 * q;
     const int col = id / CPR, cc = id % CPR;
-    gb[q] = (col < BN ? offBn[col] : 0) + cc * 2;
+    gb[q] = (col < BN ? offBn[col] : 0) + cc * 4;
     rb_row[q] = col < BN ? col : BN;
-    lb[q] = rb_row[q] * PK + cc * 2;
+    lb[q] = rb_row[q] * PK + cc * 4;
   }
   const bool lead = (tid % CPR) == 0;
 
@@ -623,7 +637,7 @@ __global__ __launch_bounds__(256) void k_gemm_h(const c64* __restrict__ A, const
   floatx4 accr[TM][TN], acci[TM][TN];
   zero_acc<mfma_t<float>, TM, TN>(accr, acci);
 
-  float4 ra[ACH], rb[BCH];
+  floatx4 ra[ACH][2], rb[BCH][2];
   auto load_tile = [&](uint32_t kt) {
     int32_t ka, kb;
     if (ktab) {
@@ -633,44 +647,80 @@ __global__ __launch_bounds__(256) void k_gemm_h(const c64* __restrict__ A, const
       group_offsets(g.K, kt * BKT, ka, kb);
     }
 #pragma unroll
-    for (int q = 0; q < ACH; ++q) ra[q] = *reinterpret_cast<const float4*>(A + ga[q] + ka);
+    for (int q = 0; q < ACH; ++q)
 #pragma unroll
-    for (int q = 0; q < BCH; ++q) rb[q] = *reinterpret_cast<const float4*>(B + gb[q] + kb);
+      for (int h = 0; h < 2; ++h) ra[q][h] = *reinterpret_cast<const floatx4*>(A + ga[q] + ka + 2 * h);
+#pragma unroll
+    for (int q = 0; q < BCH; ++q)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) rb[q][h] = *reinterpret_cast<const floatx4*>(B + gb[q] + kb + 2 * h);
   };
-  // Scale, split and store one chunk (2 complex) of a row into the planes.
-  auto split_store = [&](_Float16* p0, _Float16* p1, _Float16* p2, _Float16* p3, int at, const float4& v,
-                         int* srow, int row, bool lead_lane) {
-    float m = fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w)));
-    m = fmaxf(m, __shfl_xor(m, 8, 16));
-    m = fmaxf(m, __shfl_xor(m, 4, 16));
-    m = fmaxf(m, __shfl_xor(m, 2, 16));
-    m = fmaxf(m, __shfl_xor(m, 1, 16));
+  // Scale of a row: 2^s brings its largest magnitude into [2^14, 2^15).
+  // Magnitudes compare as integers; the maximum over the row's 8 lanes takes
+  // three DPP steps.  (Through the LDS crossbar, four steps that each waited
+  // for the last per 2 complex, and with every rounded value converted twice,
+  // the conversion was 433 instructions per K tile; 64 x 262144 x 64 took
+  // 79.4 us, now 57.5 against 52.6 at the copy rate, 64 x 32768 x 512 62.8,
+  // now 41.8.)
+  auto scale_of = [](const floatx4 (&v)[2]) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float x = v[h][r];
+        m = max(m, __builtin_bit_cast(uint32_t, x) & 0x7fffffffu);
+      }
+    m = max(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x141, 0xf, 0xf, true));   // l and 7 - l
+    m = max(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0x4e, 0xf, 0xf, true));    // quad 2, 3, 0, 1
+    m = max(m, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)m, 0xb1, 0xf, 0xf, true));    // quad 1, 0, 3, 2
     int e = 0;
-    (void)frexpf(m, &e);
-    const int sc = m > 0.f ? 15 - e : 0;         // max * 2^sc in [2^14, 2^15)
-    const float xr0 = ldexpf(v.x, sc), xi0 = ldexpf(v.y, sc), xr1 = ldexpf(v.z, sc), xi1 = ldexpf(v.w, sc);
-    half2v hr, lr, hi, li2;
-    hr.x = (_Float16)xr0;
-    hr.y = (_Float16)xr1;
-    hi.x = (_Float16)xi0;
-    hi.y = (_Float16)xi1;
-    lr.x = (_Float16)(xr0 - (float)hr.x);
-    lr.y = (_Float16)(xr1 - (float)hr.y);
-    li2.x = (_Float16)(xi0 - (float)hi.x);
-    li2.y = (_Float16)(xi1 - (float)hi.y);
-    *reinterpret_cast<half2v*>(p0 + at) = hr;
-    *reinterpret_cast<half2v*>(p1 + at) = lr;
-    *reinterpret_cast<half2v*>(p2 + at) = hi;
-    *reinterpret_cast<half2v*>(p3 + at) = li2;
-    if (lead_lane) srow[row] = sc;
+    (void)frexpf(__builtin_bit_cast(float, m), &e);
+    return m != 0 ? 15 - e : 0;
+  };
+  // Splits and stores one unit (4 complex) of a row into the planes.
+  auto split_store = [&](_Float16* p0, _Float16* p1, _Float16* p2, _Float16* p3, int at, const floatx4 (&v)[2],
+                         int sc) {
+    uint2v hr, lr, hi, lo;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      floatx2 x, y;
+      x.x = ldexpf(v[h][0], sc);
+      y.x = ldexpf(v[h][1], sc);
+      x.y = ldexpf(v[h][2], sc);
+      y.y = ldexpf(v[h][3], sc);
+      hr[h] = pack16(x);
+      hi[h] = pack16(y);
+      lr[h] = pack16(rest16(hr[h], x));
+      lo[h] = pack16(rest16(hi[h], y));
+    }
+    *reinterpret_cast<uint2v*>(p0 + at) = hr;
+    *reinterpret_cast<uint2v*>(p1 + at) = lr;
+    *reinterpret_cast<uint2v*>(p2 + at) = hi;
+    *reinterpret_cast<uint2v*>(p3 + at) = lo;
+  };
+  auto negate = [](const half8& x) {
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    return __builtin_bit_cast(half8, __builtin_bit_cast(u4, x) ^ 0x80008000u);
   };
 
   load_tile(0);
   for (uint32_t kt = 0; kt < ntiles; ++kt) {
+    int ea[ACH], eb[BCH];
 #pragma unroll
-    for (int q = 0; q < ACH; ++q) split_store(Ap[0], Ap[1], Ap[2], Ap[3], la[q], ra[q], sA, ra_row[q], lead);
+    for (int q = 0; q < ACH; ++q) ea[q] = scale_of(ra[q]);
 #pragma unroll
-    for (int q = 0; q < BCH; ++q) split_store(Bp[0], Bp[1], Bp[2], Bp[3], lb[q], rb[q], sB, rb_row[q], lead);
+    for (int q = 0; q < BCH; ++q) eb[q] = scale_of(rb[q]);
+#pragma unroll
+    for (int q = 0; q < ACH; ++q) split_store(Ap[0], Ap[1], Ap[2], Ap[3], la[q], ra[q], ea[q]);
+#pragma unroll
+    for (int q = 0; q < BCH; ++q) split_store(Bp[0], Bp[1], Bp[2], Bp[3], lb[q], rb[q], eb[q]);
+    if (lead) {
+#pragma unroll
+      for (int q = 0; q < ACH; ++q) sA[ra_row[q]] = ea[q];
+#pragma unroll
+      for (int q = 0; q < BCH; ++q) sB[rb_row[q]] = eb[q];
+    }
     __syncthreads();
     if (kt + 1 < ntiles) load_tile(kt + 1);
     half8 a[TM][4], an[TM][2], b[TN][4];
@@ -679,8 +729,8 @@ __global__ __launch_bounds__(256) void k_gemm_h(const c64* __restrict__ A, const
       const int at = (wm + 16 * i + li) * PK + 8 * lk;
 #pragma unroll
       for (int pl = 0; pl < 4; ++pl) a[i][pl] = *reinterpret_cast<const half8*>(&Ap[pl][at]);
-      an[i][0] = -a[i][2];
-      an[i][1] = -a[i][3];
+      an[i][0] = negate(a[i][2]);
+      an[i][1] = negate(a[i][3]);
     }
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
