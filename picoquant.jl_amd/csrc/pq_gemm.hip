@@ -149,6 +149,7 @@ __global__ __launch_bounds__(256) void k_gemm(const C* __restrict__ A, const C* 
   __shared__ int32_t offAm[BM], offBn[BN];
   __shared__ int32_t offAk[KTAB_MAX], offBk[KTAB_MAX];
 
+  PQ_TOUCH(g.M, g.N, g.K, g.L);
   const uint32_t Mt = g.M.total, Nt = g.N.total, Kt = g.K.total;
   uint32_t tile_x, tile_y;
   xcd_tile(tile_x, tile_y);
@@ -316,6 +317,7 @@ __global__ __launch_bounds__(256) void k_gemm2(const C* __restrict__ A, const C*
   __shared__ int32_t offAm[BM], offCm[BM], offBn[BN], offCn[BN];
   __shared__ int32_t offAk[KT_MAX], offBk[KT_MAX];
 
+  PQ_TOUCH(g.M, g.N, g.K, g.L);
   const uint32_t Mt = g.M.total, Nt = g.N.total, Kt = g.K.total;
   uint32_t tile_x, tile_y;
   xcd_tile(tile_x, tile_y);
@@ -490,7 +492,7 @@ hipError_t launch_tile(const C* A, const C* B, C* Out, const GemmArgs& g, hipStr
     // K tile depth: the deepest of 32 / 16 / 8 (within the tile's LDS
     // budget) that divides the first (contiguous) K mode, so a tile never
     // straddles two runs.
-    const uint32_t k0ext = g.K.nmodes > 0 ? g.K.ext[0].d : 0;
+    const uint32_t k0ext = g.K.nmodes > 0 ? g.K.m[0].ext.d : 0;
     if (g.contig && k0ext > 0) {
       if (k0ext % BKF == 0) {
         hipLaunchKernelGGL((k_gemm2<C, BM, BN, WGM, BKF>), grid, dim3(256), 0, s, A, B, Out, g);
@@ -572,6 +574,7 @@ __global__ __launch_bounds__(256) void k_gemm_h(const c64* __restrict__ A, const
   __shared__ int32_t offAm[BM], offCm[BM], offBn[BN], offCn[BN];
   __shared__ int32_t offAk[KT_MAX], offBk[KT_MAX];
 
+  PQ_TOUCH(g.M, g.N, g.K, g.L);
   const uint32_t Mt = g.M.total, Nt = g.N.total, Kt = g.K.total;
   uint32_t tile_x, tile_y;
   xcd_tile(tile_x, tile_y);
@@ -857,7 +860,7 @@ hipError_t launch_gemm(const C* A, const C* B, C* Out, const GemmArgs& g, hipStr
 }
 
 bool gemm16_applicable(const GemmArgs& g) {
-  return g.contig && g.K.nmodes > 0 && g.K.ext[0].d % 32 == 0 && g.K.total <= GEMM_K_MAX &&
+  return g.contig && g.K.nmodes > 0 && g.K.m[0].ext.d % 32 == 0 && g.K.total <= GEMM_K_MAX &&
          g.L.total >= 1 && g.L.total <= 65535;
 }
 

@@ -31,6 +31,7 @@ template <typename C, int KP>
 __global__ __launch_bounds__(256) void k_stream(const C* __restrict__ X, const C* __restrict__ Y,
                                                 C* __restrict__ Out, StreamArgs a) {
   extern __shared__ unsigned char smem_raw[];
+  PQ_TOUCH(a.M, a.K, a.N, a.L);
   const uint32_t Kt = a.K.total, Nt = a.N.total, Mt = a.M.total;
   {
     int64_t ox, oy, oc;
@@ -96,6 +97,7 @@ __global__ __launch_bounds__(256) void k_stream(const C* __restrict__ X, const C
 template <typename C>
 __global__ __launch_bounds__(256) void k_generic(const C* __restrict__ A, const C* __restrict__ B,
                                                  C* __restrict__ Out, GenArgs a) {
+  PQ_TOUCH(a.M, a.N, a.K, a.L);
   const uint32_t Mt = a.M.total, Nt = a.N.total, Kt = a.K.total;
   const uint64_t total = (uint64_t)Mt * Nt;
   {
@@ -283,6 +285,7 @@ __global__ __launch_bounds__(256) void k_copy_bits(const C* __restrict__ In, C* 
 template <typename C>
 __global__ __launch_bounds__(256) void k_multi(const MultiDesc* __restrict__ descs, int64_t group) {
   const MultiDesc& d = descs[blockIdx.y];
+  PQ_TOUCH(d.M, d.N, d.K, d.L);
   if (blockIdx.z >= d.L.total) return;
   int64_t oa, ob, oc;
   batch_offsets(d.L, blockIdx.z, oa, ob, oc);

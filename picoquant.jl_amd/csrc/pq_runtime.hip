@@ -53,12 +53,14 @@ bool fill_group(Group& g, const std::vector<Mode>& modes) {
   if ((int)modes.size() > PQ_MAX_MODES) return false;
   memset(&g, 0, sizeof(g));
   g.nmodes = (int)modes.size();
+  g.pow2 = 1;
   uint64_t total = 1;
   for (size_t j = 0; j < modes.size(); ++j) {
     if (modes[j].s0 >= (1ll << 31) || modes[j].s1 >= (1ll << 31)) return false;
-    g.ext[j] = make_fdiv((uint32_t)modes[j].ext);
-    g.s0[j] = (int32_t)modes[j].s0;
-    g.s1[j] = (int32_t)modes[j].s1;
+    g.m[j].ext = make_fdiv((uint32_t)modes[j].ext);
+    g.m[j].s0 = (int32_t)modes[j].s0;
+    g.m[j].s1 = (int32_t)modes[j].s1;
+    if (modes[j].ext & (modes[j].ext - 1)) g.pow2 = 0;
     total *= (uint64_t)modes[j].ext;
   }
   if (total >= (1ull << 31)) return false;
