@@ -12,6 +12,7 @@
 //              (materialises permuted / sliced views).
 #include "pq_internal.h"
 
+#include <algorithm>
 #include <cstring>
 #include <type_traits>
 
@@ -124,11 +125,22 @@ __global__ __launch_bounds__(256) void k_generic(const C* __restrict__ A, const 
 }
 
 // ---------------------------------------------------------------- k_reduce
-// Phase 1: workgroup b sums its K chunk for every output; partials[b*MN + o].
-template <typename C>
+// Phase 1: workgroup b sums its K chunk for all outputs at once (at most TM x
+// TN of them, padded to powers of two): every K value reads each operand row
+// once.  partials[b * MN + o]; with a single workgroup the outputs
+// themselves.
+// With power-of-two K modes an offset is the sum of its index bits': a lane's
+// own 8 bits are decoded once, and the wave's 64 lanes decode the uniform
+// parts of its next 64 steps together (decoded per step on the scalar unit,
+// 23 modes held the loop at 68 us where the loads alone take 46).
+// Bound: HBM for long K (2^23 against 2^23 complex128: 180 us before, 53.5
+// now at 53 for the bytes), two launches for short (a call on 2^14 x 2^13
+// elements closed over 2^13: 39 us on 2 workgroups, 15 on 16).
+template <typename C, int TM, int TN>
 __global__ __launch_bounds__(256) void k_reduce_partial(const C* __restrict__ A, const C* __restrict__ B,
-                                                        C* __restrict__ partials, GenArgs a) {
-  __shared__ C red[256];
+                                                        C* __restrict__ partials, C* __restrict__ Out, GenArgs a) {
+  __shared__ C red[4][TM * TN];
+  PQ_TOUCH(a.K, a.M, a.N, a.L);
   const uint32_t Mt = a.M.total, Nt = a.N.total, Kt = a.K.total;
   const uint32_t MN = Mt * Nt;
   {
@@ -136,33 +148,117 @@ __global__ __launch_bounds__(256) void k_reduce_partial(const C* __restrict__ A,
     batch_offsets(a.L, blockIdx.z, oa, ob, oc);
     A += oa;
     B += ob;
+    Out += oc;
   }
-  partials += (size_t)blockIdx.z * gridDim.x * MN;
-  const uint32_t chunk = (Kt + gridDim.x - 1) / gridDim.x;
+  int32_t om[TM], on[TN];
+#pragma unroll
+  for (int m = 0; m < TM; ++m) {
+    int32_t oc = 0;
+    om[m] = 0;
+    if (m < (int)Mt) group_offsets(a.M, (uint32_t)m, om[m], oc);
+  }
+#pragma unroll
+  for (int n = 0; n < TN; ++n) {
+    int32_t oc = 0;
+    on[n] = 0;
+    if (n < (int)Nt) group_offsets(a.N, (uint32_t)n, on[n], oc);
+  }
+  const uint32_t chunk = ((Kt + gridDim.x - 1) / gridDim.x + 255) / 256 * 256;
   const uint32_t k0 = blockIdx.x * chunk;
   const uint32_t k1 = min(Kt, k0 + chunk);
-  for (uint32_t o = 0; o < MN; ++o) {
-    uint32_t m = o % Mt, n = o / Mt;
-    int32_t oa, oc1, ob, oc2;
-    group_offsets(a.M, m, oa, oc1);
-    group_offsets(a.N, n, ob, oc2);
-    C acc = czero<C>();
-    for (uint32_t k = k0 + threadIdx.x; k < k1; k += blockDim.x) {
-      int32_t ka, kb;
-      group_offsets(a.K, k, ka, kb);
-      cfma(acc, A[oa + ka], B[ob + kb]);
-    }
-    red[threadIdx.x] = acc;
-    __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-      if ((int)threadIdx.x < w) {
-        red[threadIdx.x].x += red[threadIdx.x + w].x;
-        red[threadIdx.x].y += red[threadIdx.x + w].y;
+  C acc[TM][TN];
+#pragma unroll
+  for (int m = 0; m < TM; ++m)
+#pragma unroll
+    for (int n = 0; n < TN; ++n) acc[m][n] = czero<C>();
+  // U values of K at a time, so that their loads are in flight together.
+  // Rows past the operands' extents read the first row; their sums are not
+  // stored.
+  constexpr int U = TM + TN <= 4 ? 4 : (TM + TN <= 8 ? 2 : 1);
+  auto add = [&](const int32_t (&ka)[U], const int32_t (&kb)[U], int live) {
+    C x[U][TM], y[U][TN];
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (u < live) {
+#pragma unroll
+        for (int m = 0; m < TM; ++m) x[u][m] = A[om[m] + ka[u]];
+#pragma unroll
+        for (int n = 0; n < TN; ++n) y[u][n] = B[on[n] + kb[u]];
       }
-      __syncthreads();
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (u < live) {
+#pragma unroll
+        for (int m = 0; m < TM; ++m)
+#pragma unroll
+          for (int n = 0; n < TN; ++n) cfma(acc[m][n], x[u][m], y[u][n]);
+      }
+  };
+  if (a.K.pow2 && Kt >= 256) {
+    // a wave's lanes decode the uniform parts of 64 steps in one go
+    int32_t la, lb;
+    group_offsets(a.K, threadIdx.x, la, lb);
+    for (uint32_t kb = k0; kb < k1; kb += 256 * 64) {
+      const uint32_t mine = kb + 256 * (threadIdx.x & 63);
+      int32_t va = 0, vb = 0;
+      if (mine < k1) group_offsets(a.K, mine, va, vb);
+      const int steps = (int)min(64u, (k1 - kb) / 256);
+      for (int i = 0; i < steps; i += U) {
+        int32_t ka[U], kq[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int t = min(i + u, steps - 1);
+          ka[u] = __builtin_amdgcn_readlane(va, t) + la;
+          kq[u] = __builtin_amdgcn_readlane(vb, t) + lb;
+        }
+        if (i + U <= steps)
+          add(ka, kq, U);
+        else
+          add(ka, kq, steps - i);
+      }
     }
-    if (threadIdx.x == 0) partials[(size_t)blockIdx.x * MN + o] = red[0];
-    __syncthreads();
+  } else {
+    for (uint32_t k = k0 + threadIdx.x; k < k1; k += 256 * U) {
+      int32_t ka[U], kq[U];
+      int live = 0;
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        ka[u] = kq[u] = 0;
+        if (k + 256 * u < k1) {
+          group_offsets(a.K, k + 256 * u, ka[u], kq[u]);
+          live = u + 1;
+        }
+      }
+      add(ka, kq, live);
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < TM; ++m)
+#pragma unroll
+    for (int n = 0; n < TN; ++n) {
+      for (int w = 32; w > 0; w >>= 1) {
+        acc[m][n].x += __shfl_xor(acc[m][n].x, w);
+        acc[m][n].y += __shfl_xor(acc[m][n].y, w);
+      }
+      if ((threadIdx.x & 63) == 0) red[threadIdx.x / 64][m + TM * n] = acc[m][n];
+    }
+  __syncthreads();
+  const int t = (int)threadIdx.x, m = t % TM, n = t / TM;
+  if (t < TM * TN && m < (int)Mt && n < (int)Nt) {
+    C v = red[0][t];
+#pragma unroll
+    for (int w = 1; w < 4; ++w) {
+      v.x += red[w][t].x;
+      v.y += red[w][t].y;
+    }
+    if (gridDim.x == 1) {
+      int32_t oa, oc1, ob, oc2;
+      group_offsets(a.M, (uint32_t)m, oa, oc1);
+      group_offsets(a.N, (uint32_t)n, ob, oc2);
+      Out[oc1 + oc2] = v;
+    } else {
+      partials[((size_t)blockIdx.z * gridDim.x + blockIdx.x) * MN + m + Mt * n] = v;
+    }
   }
 }
 
@@ -517,19 +613,39 @@ hipError_t launch_generic(const C* A, const C* B, C* Out, const GenArgs& a, hipS
   return hipGetLastError();
 }
 
-int reduce_blocks_for(uint32_t ktotal) {
-  uint32_t b = ktotal / 4096;
-  if (b < 1) b = 1;
-  if (b > 2048) b = 2048;
-  return (int)b;
+int reduce_blocks_for(uint32_t ktotal, uint32_t batch) {
+  // 4096 values of K per workgroup (16 per lane) and at most 2048 workgroups;
+  // fewer values, down to 512, while that keeps the device short of 2048
+  const uint32_t least = ktotal / 4096, fill = std::min(ktotal / 512, 2048u / std::max(batch, 1u));
+  return (int)std::min(std::max(std::max(least, fill), 1u), 2048u);
+}
+
+template <typename C, int TM, int TN>
+static void reduce_partial(const C* A, const C* B, C* Out, const GenArgs& a, C* partials, int nblocks, hipStream_t s) {
+  hipLaunchKernelGGL((k_reduce_partial<C, TM, TN>), dim3(nblocks, 1, a.L.total), dim3(256), 0, s, A, B, partials, Out,
+                     a);
 }
 
 template <typename C>
 hipError_t launch_reduce(const C* A, const C* B, C* Out, const GenArgs& a, C* partials, int nblocks,
                          hipStream_t s) {
-  hipLaunchKernelGGL((k_reduce_partial<C>), dim3(nblocks, 1, a.L.total), dim3(256), 0, s, A, B, partials, a);
+  auto log2up = [](uint32_t v) {
+    int l = 0;
+    while ((1u << l) < v) ++l;
+    return l;
+  };
+  const int lm = log2up(a.M.total), ln = log2up(a.N.total);
+  switch (lm * 8 + ln) {
+#define PQ_CASE(LM, LN) \
+  case LM * 8 + LN: reduce_partial<C, 1 << LM, 1 << LN>(A, B, Out, a, partials, nblocks, s); break;
+    PQ_CASE(0, 0) PQ_CASE(0, 1) PQ_CASE(0, 2) PQ_CASE(0, 3) PQ_CASE(0, 4) PQ_CASE(1, 0) PQ_CASE(1, 1) PQ_CASE(1, 2)
+    PQ_CASE(1, 3) PQ_CASE(2, 0) PQ_CASE(2, 1) PQ_CASE(2, 2) PQ_CASE(2, 3) PQ_CASE(3, 0) PQ_CASE(3, 1) PQ_CASE(3, 2)
+    PQ_CASE(4, 0)
+#undef PQ_CASE
+    default: return hipErrorInvalidValue;
+  }
   hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
+  if (e != hipSuccess || nblocks == 1) return e;
   hipLaunchKernelGGL((k_reduce_final<C>), dim3(a.M.total * a.N.total, 1, a.L.total), dim3(256), 0, s, partials,
                      Out, a, nblocks);
   return hipGetLastError();

@@ -386,6 +386,40 @@ static bool stream_fits(uint64_t Kt, uint64_t Ny, size_t esize) {
   return Kt <= PQ_STREAM_KMAX && Kt * Ny <= PQ_STREAM_YMAX && smem <= 48 * 1024;
 }
 
+// The order of the summed modes of a long reduction (free) so that a wave
+// reads whole lines of both operands: the factors of two by three in turn
+// from the smallest strides of A and of B (8 elements each way per wave; in
+// A's order alone every element of a differently ordered B is a line of its
+// own: 106 us for 2^23 complex128 in two unlike orders, 53 in this one; two
+// like orders do not care).  Not with odd extents or more bits than modes fit.
+static void interleave_k(std::vector<Mode>& K) {
+  std::vector<Mode> bits;
+  for (const Mode& m : K) {
+    if (m.ext & (m.ext - 1)) return;
+    for (int64_t k = 1; k < m.ext; k <<= 1) bits.push_back({2, m.s0 * k, m.s1 * k});
+  }
+  if (bits.size() > PQ_MAX_MODES) return;
+  std::vector<size_t> by[2];
+  for (int side = 0; side < 2; ++side) {
+    for (size_t i = 0; i < bits.size(); ++i) by[side].push_back(i);
+    std::stable_sort(by[side].begin(), by[side].end(), [&](size_t x, size_t y) {
+      return side ? bits[x].s1 < bits[y].s1 : bits[x].s0 < bits[y].s0;
+    });
+  }
+  std::vector<char> used(bits.size(), 0);
+  size_t at[2] = {0, 0};
+  std::vector<Mode> out;
+  while (out.size() < bits.size())
+    for (int side = 0; side < 2; ++side)
+      for (int n = 0; n < 3 && at[side] < bits.size(); ++at[side])
+        if (!used[by[side][at[side]]]) {
+          used[by[side][at[side]]] = 1;
+          out.push_back(bits[by[side][at[side]]]);
+          ++n;
+        }
+  K = merge_modes(out);
+}
+
 int resolve_step(pq_ctx* c, StepSpec& s, size_t esize) {
   s.Mt = s.Nt = s.Kt = 1;
   for (auto& m : s.M) s.Mt *= m.ext;
@@ -455,6 +489,7 @@ int resolve_step(pq_ctx* c, StepSpec& s, size_t esize) {
         }
   } else if (kc == PQ_KC_REDUCE) {
     if (Mt * Nt > 16) return fail(c, PQ_ERR_UNSUPPORTED, "reduce kernel needs M*N <= 16");
+    if (Kt >= 4096) interleave_k(s.K);
   } else if (kc != PQ_KC_GENERIC) {
     return fail(c, PQ_ERR_UNSUPPORTED, "kernel class not available for this shape");
   }
@@ -531,7 +566,7 @@ int prepare_contract(pq_ctx* c, const Tensor& A, int ra, const int32_t* ia, cons
 size_t step_scratch_bytes(const StepSpec& s, size_t esize) {
   if (s.kc == PQ_KC_GEMM && s.splitk > 1) return (size_t)s.splitk * s.Mt * s.Nt * esize;
   if (s.kc != PQ_KC_REDUCE) return 0;
-  return (size_t)reduce_blocks_for((uint32_t)s.Kt) * s.Mt * s.Nt * s.L.total * esize;
+  return (size_t)reduce_blocks_for((uint32_t)s.Kt, s.L.total) * s.Mt * s.Nt * s.L.total * esize;
 }
 
 template <typename C>
@@ -654,7 +689,7 @@ static int launch_typed(pq_ctx* c, const C* pa, const C* pb, C* pc, const StepSp
     ga.L = s.L;
     if (s.kc == PQ_KC_REDUCE) {
       ProfScope ps(c, PQ_KC_REDUCE, alg_bytes, alg_flops);
-      e = launch_reduce<C>(pa, pb, pc, ga, reinterpret_cast<C*>(scratch), reduce_blocks_for((uint32_t)s.Kt),
+      e = launch_reduce<C>(pa, pb, pc, ga, reinterpret_cast<C*>(scratch), reduce_blocks_for((uint32_t)s.Kt, s.L.total),
                            c->stream);
     } else {
       ProfScope ps(c, PQ_KC_GENERIC, alg_bytes, alg_flops);

@@ -192,3 +192,22 @@ def test_error_paths(ctx):
     ctx.free(h)
     with pytest.raises(KeyError):
         ctx.free(h)
+
+
+@pytest.mark.parametrize("M,N", [(1, 1), (2, 1), (1, 3), (4, 4), (5, 3), (3, 5), (16, 1), (1, 9), (2, 8), (7, 2)])
+@pytest.mark.parametrize("K", [65, 255, 256, 511, 512, 1000, 4096, 3 * 2 ** 12, 2 ** 17, 100003])
+def test_reduce_outputs_and_extents(ctx, M, N, K):
+    """Every padded output shape of the split reduction, one workgroup and
+    many, summed extents around its workgroup size and not powers of two;
+    summed axes in another order in B."""
+    rng = np.random.default_rng(M * 100 + N + K)
+    if K & (K - 1) == 0:
+        q = K.bit_length() - 1
+        perm = rng.permutation(q)
+        A = rand(rng, [2] * q + [M], ctx.np_dtype)
+        B = rand(rng, [N] + [2] * q, ctx.np_dtype)
+        ia, ib = list(range(1, q + 1)) + [-1], [-2] + [int(x) + 1 for x in perm]
+    else:
+        A, B = rand(rng, (M, K), ctx.np_dtype), rand(rng, (K, N), ctx.np_dtype)
+        ia, ib = [-1, 1], [1, -2]
+    check(ctx, A, ia, B, ib, run(ctx, A, ia, B, ib, _lib.KC_REDUCE))
