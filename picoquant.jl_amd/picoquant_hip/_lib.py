@@ -131,13 +131,19 @@ def load(required_symbols=True):
     return lib
 
 
+# Array types by length: making `c_int32 * n` anew costs as much as filling it.
+_I32 = [ct.c_int32 * max(1, n) for n in range(PQ_MAX_RANK + 1)]
+_I64 = [ct.c_int64 * max(1, n) for n in range(PQ_MAX_RANK + 1)]
+
+
 def i64arr(xs):
-    a = (ct.c_int64 * max(1, len(xs)))(*[int(x) for x in xs])
-    return a
+    n = len(xs)
+    return (_I64[n] if n <= PQ_MAX_RANK else ct.c_int64 * n)(*map(int, xs))
 
 
 def i32arr(xs):
-    return (ct.c_int32 * max(1, len(xs)))(*[int(x) for x in xs])
+    n = len(xs)
+    return (_I32[n] if n <= PQ_MAX_RANK else ct.c_int32 * n)(*map(int, xs))
 
 
 class Context:
@@ -183,10 +189,11 @@ class Context:
             host, code = np.asfortranarray(a), PQ_C64
         else:
             host, code = np.asfortranarray(a.astype(np.complex128, copy=False)), PQ_C128
-        dims = i64arr(a.shape)
         h = ct.c_int64()
-        self.check(self.lib.pq_tensor_upload(self.ptr, a.ndim, dims, host.ctypes.data_as(ct.c_void_p),
-                                             code, ct.byref(h)))
+        rc = self.lib.pq_tensor_upload(self.ptr, a.ndim, i64arr(a.shape), host.__array_interface__["data"][0], code,
+                                       ct.byref(h))
+        if rc:
+            self.check(rc)
         return h.value
 
     def shape(self, h):
@@ -213,12 +220,15 @@ class Context:
         self.check(self.lib.pq_tensor_write(self.ptr, h, host.ctypes.data_as(ct.c_void_p), code))
 
     def free(self, h):
-        self.check(self.lib.pq_tensor_free(self.ptr, h))
+        rc = self.lib.pq_tensor_free(self.ptr, h)
+        if rc:
+            self.check(rc)
 
     def contract(self, ha, ia, hb, ib):
         out = ct.c_int64()
-        self.check(self.lib.pq_contract(self.ptr, ha, len(ia), i32arr(ia), hb, len(ib), i32arr(ib),
-                                        ct.byref(out)))
+        rc = self.lib.pq_contract(self.ptr, ha, len(ia), i32arr(ia), hb, len(ib), i32arr(ib), ct.byref(out))
+        if rc:
+            self.check(rc)
         return out.value
 
     def set_plan_streams(self, n):

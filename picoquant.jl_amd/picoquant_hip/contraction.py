@@ -7,30 +7,22 @@ from .backend import record_compute_costs
 from .network import Node, new_label
 
 
-def _unique(seq):
-    seen = set()
-    out = []
-    for x in seq:
-        if x not in seen:
-            seen.add(x)
-            out.append(x)
-    return out
-
-
 def sort_indices(A: Node, B: Node):
     """src/layer2.jl:209-216: common = A ∩ B (A's order); remaining =
     (A \\ common) ∪ (B \\ common), first occurrence order."""
+    both = dict.fromkeys(A.indices)
     bset = set(B.indices)
-    common = _unique([x for x in A.indices if x in bset])
-    cset = set(common)
-    rem = _unique([x for x in A.indices if x not in cset] + [x for x in B.indices if x not in cset])
-    return common, rem
+    common = [x for x in both if x in bset]
+    both.update(dict.fromkeys(B.indices))
+    for x in common:
+        del both[x]
+    return common, list(both)
 
 
 def create_ncon_indices(A: Node, B: Node, common, uncommon):
     """src/layer2.jl:226-240: summed indices get +1.., open ones -1.."""
-    m = {x: i + 1 for i, x in enumerate(common)}
-    m.update({x: -(i + 1) for i, x in enumerate(uncommon)})
+    m = dict(zip(common, range(1, len(common) + 1)))
+    m.update(zip(uncommon, range(-1, -len(uncommon) - 1, -1)))
     return [m[x] for x in A.indices], [m[x] for x in B.indices]
 
 

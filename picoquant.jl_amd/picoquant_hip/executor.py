@@ -562,11 +562,11 @@ class Plan:
 
     def _shaped(self, buf):
         n = int(np.prod(self.out_shape)) if self.out_shape else 1
-        z = buf[0::2] + 1j * buf[1::2]
+        z = buf.view(np.complex128)
         if self.n_bitstrings is None:
             return z.reshape(self.out_shape, order="F")
-        return np.stack([z[b * n:(b + 1) * n].reshape(self.out_shape, order="F")
-                         for b in range(self.n_bitstrings)])
+        nb = self.n_bitstrings
+        return np.ascontiguousarray(np.moveaxis(z[:nb * n].reshape(tuple(self.out_shape) + (nb,), order="F"), -1, 0))
 
     def set_bitstrings(self, bitstrings):
         """Rewrite the output batch in place (pq_plan_set_bitstrings): the
@@ -581,10 +581,13 @@ class Plan:
         bitstrings = list(bitstrings)
         if len(bitstrings) != self.n_bitstrings:
             raise ValueError(f"the plan computes {self.n_bitstrings} bitstrings per run")
-        data, _ = output_batch(self.network, bitstrings)
-        if set(data) != set(self.batch_handles):
+        n = self.network.number_qubits
+        if any(len(b) != n for b in bitstrings):
+            raise ValueError(f"every bitstring needs {n} characters")
+        words = bitstring_words(self.network, bitstrings)
+        if {node for node, _ in closed_output_qubits(self.network)} != set(self.batch_handles):
             raise ValueError("the bitstrings close other outputs than the plan's")
-        return bitstring_words(self.network, bitstrings)
+        return words
 
     def run(self, bitstrings=None):
         """pq_plan_run: set the bitstrings (if given), run once (graph) and
@@ -743,7 +746,16 @@ def bitstring_words(network, bitstrings):
     if any(i > 63 for _, i in closed):
         raise ValueError("bitstring words hold at most 64 qubits")
     words = (ct.c_uint64 * len(bitstrings))()
+    last = max((i for _, i in closed), default=-1)
+    opened = sorted(set(range(last + 1)) - {i for _, i in closed})
     for b, bits in enumerate(bitstrings):
+        if type(bits) is str and 0 <= last < len(bits):
+            digits = bits[:last + 1]
+            for i in opened:
+                digits = digits[:i] + "0" + digits[i + 1:]
+            if not digits.strip("01"):                     # nothing but 0 and 1: one conversion for all qubits
+                words[b] = int(digits[::-1], 2)
+                continue
         w = 0
         for _, i in closed:
             if bits[i] not in "01":

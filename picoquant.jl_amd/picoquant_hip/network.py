@@ -91,14 +91,15 @@ def decompose_gate(gate_data, threshold=1e-15):
 
 
 def _rewire(network, node_label, input_index, output_index, qubit):
-    network.edges[output_index] = Edge(node_label, network.edges[input_index].dst, qubit)
-    dst = network.edges[input_index].dst
+    edge = network.edges[input_index]
+    dst = edge.dst
+    network.edges[output_index] = Edge(node_label, dst, qubit)
     if dst is not None:
         out_node = network.nodes[dst]
         for i, x in enumerate(out_node.indices):
             if x == input_index:
                 out_node.indices[i] = output_index
-    network.edges[input_index].dst = node_label
+    edge.dst = node_label
 
 
 def add_gate(network, gate_data, target_qubits, decompose=False):
@@ -177,7 +178,7 @@ def gate_matrix_to_tensor(U):
     is G[in_1..in_k, out_1..out_k] = U[out, in]."""
     U = np.asarray(U, dtype=np.complex128)
     k = int(round(math.log2(U.shape[0])))
-    return np.reshape(np.ascontiguousarray(U.T), (2,) * (2 * k), order="F")
+    return U.flatten().reshape((2,) * (2 * k), order="F")      # element in + 2^k out = U[out, in]
 
 
 def network_from_gates(n_qubits, gates, backend=None, decompose=False):

@@ -232,3 +232,25 @@ def test_bitstring_words_for_the_c_abi():
         assert words[b] == want
     with pytest.raises(ValueError):
         bitstring_words(tn, ["1x0x11x0x"])
+
+
+@pytest.mark.parametrize("config", ["x0x1x", "0101x", "x1010", "01010"])
+def test_bitstring_words_any_sequence_of_characters(config):
+    """A string and a list of its characters give the same words, whatever
+    stands at the open qubits; other characters at closed ones are refused."""
+    from picoquant_hip.executor import bitstring_words
+    tn = P.TensorNetworkCircuit.create(5, RecordingBackend())
+    P.add_input(tn, "00000")
+    P.add_output(tn, config)
+    closed = [i for i, c in enumerate(config) if c != "x"]
+    batch = ["01x10", "11111", "00000", "1_101", "10 01"]
+    batch = ["".join(c if i not in closed or c in "01" else "1" for i, c in enumerate(b)) for b in batch]
+    want = [sum(int(b[i]) << i for i in closed) for b in batch]
+    assert list(bitstring_words(tn, batch)) == want
+    assert list(bitstring_words(tn, [list(b) for b in batch])) == want
+    for bad in ("_", "x", "2", " "):
+        for b in ("0" * closed[0] + bad + "0" * (4 - closed[0]), "1" * closed[-1] + bad + "1" * (4 - closed[-1])):
+            with pytest.raises(ValueError):
+                bitstring_words(tn, [b])
+    with pytest.raises(IndexError):
+        bitstring_words(tn, ["0" * closed[-1]])
