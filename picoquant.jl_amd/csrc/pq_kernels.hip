@@ -21,14 +21,32 @@ namespace {
 template <typename C>
 __device__ __forceinline__ C czero() { C r; r.x = 0; r.y = 0; return r; }
 
-template <typename C>
-__device__ __forceinline__ C ldg(const C* p) { return *p; }
+// One element, past the caches when NT (non-temporal).
+template <bool NT, typename C>
+__device__ __forceinline__ C load_one(const C* p) {
+  typedef decltype(C::x) V __attribute__((ext_vector_type(2)));
+  if constexpr (!NT) return *p;
+  return __builtin_bit_cast(C, __builtin_nontemporal_load(reinterpret_cast<const V*>(p)));
+}
+template <bool NT, typename C>
+__device__ __forceinline__ void store_one(C* p, const C& v) {
+  typedef decltype(C::x) V __attribute__((ext_vector_type(2)));
+  if constexpr (NT)
+    __builtin_nontemporal_store(__builtin_bit_cast(V, v), reinterpret_cast<V*>(p));
+  else
+    *p = v;
+}
 
 // ---------------------------------------------------------------- k_stream
 // The lane's first X-open index has its K values loaded before the small
 // operand is staged in LDS: those loads depend on nothing the staging writes,
 // so the kernel waits for global memory once before the barrier, not twice.
-template <typename C, int KP>
+// Bound: HBM, or the 256 MB last-level cache where X and Out fit it (7.6 TB/s
+// at 2^24 complex64).  NT: X and Out are together too large for that cache,
+// so Out (1) or both (2) pass it, and a lane takes one index instead of up
+// to 16 (launch_stream): 2^25 complex64 from three states in turn 117 -> 97
+// us, 2^26 195 -> 167.
+template <typename C, int KP, int NT>
 __global__ __launch_bounds__(256) void k_stream(const C* __restrict__ X, const C* __restrict__ Y,
                                                 C* __restrict__ Out, StreamArgs a) {
   extern __shared__ unsigned char smem_raw[];
@@ -56,7 +74,7 @@ __global__ __launch_bounds__(256) void k_stream(const C* __restrict__ X, const C
     int32_t ox;
     group_offsets(a.M, m, ox, oc);
 #pragma unroll
-    for (int k = 0; k < KP; ++k) xv[k] = (k < (int)Kt) ? ldg(X + ox + xk[k]) : czero<C>();
+    for (int k = 0; k < KP; ++k) xv[k] = (k < (int)Kt) ? load_one<NT == 2>(X + ox + xk[k]) : czero<C>();
   }
   C* ys = reinterpret_cast<C*>(smem_raw);                              // [KP][Nt]
   int32_t* cn = reinterpret_cast<int32_t*>(ys + (size_t)KP * Nt);      // [Nt]
@@ -82,14 +100,14 @@ __global__ __launch_bounds__(256) void k_stream(const C* __restrict__ X, const C
       int32_t ox;
       group_offsets(a.M, m, ox, oc);
 #pragma unroll
-      for (int k = 0; k < KP; ++k) xv[k] = (k < (int)Kt) ? ldg(X + ox + xk[k]) : czero<C>();
+      for (int k = 0; k < KP; ++k) xv[k] = (k < (int)Kt) ? load_one<NT == 2>(X + ox + xk[k]) : czero<C>();
     }
     for (uint32_t n = 0; n < Nt; ++n) {
       C acc = czero<C>();
       const C* yc = ys + (size_t)n * KP;
 #pragma unroll
       for (int k = 0; k < KP; ++k) cfma(acc, xv[k], yc[k]);
-      Out[oc + cn[n]] = acc;
+      store_one<NT != 0>(Out + oc + cn[n], acc);
     }
   }
 }
@@ -594,12 +612,23 @@ hipError_t launch_stream(const C* X, const C* Y, C* Out, const StreamArgs& a, hi
   int KP = 1;
   while ((uint32_t)KP < Kt) KP <<= 1;
   size_t smem = (size_t)KP * Nt * sizeof(C) + (size_t)Nt * 4;
-  unsigned grid = grid_for(a.M.total, 256, a.L.total > 1 ? 1024 : 4096);
-  switch (KP) {
-#define PQ_CASE(P) \
-  case P: hipLaunchKernelGGL((k_stream<C, P>), dim3(grid, 1, a.L.total), dim3(256), smem, s, X, Y, Out, a); break;
+  // X and Out pass the caches when they are well over the last level's 256
+  // MB.  Measured a gate at a time, each on the last one's result: 256 MB
+  // together 35-43 us with the caches, 47-54 without; 512 MB 93-109 and
+  // 92-101; 1 GB 193-220 and 167-196.  X only where the lanes' loads cover its
+  // lines at once (the lowest bit summed, 512 MB: 97 us with X cached, 102
+  // without).  More than 4096 workgroups are an eighth slower where the
+  // caches serve (each stages Y) and a tenth faster past them.
+  const bool past = (double)a.M.total * a.L.total * (Kt + Nt) * sizeof(C) > 384.0 * (1 << 20);
+  const int nt = !past ? 0 : (a.M.m[0].s0 == 1 ? 2 : 1);
+  const dim3 grid(grid_for(a.M.total, 256, a.L.total > 1 ? 1024 : (past ? 65536 : 4096)), 1, a.L.total), block(256);
+  switch (KP * 4 + nt) {
+#define PQ_CASE2(P, NT) \
+  case P * 4 + NT: hipLaunchKernelGGL((k_stream<C, P, NT>), grid, block, smem, s, X, Y, Out, a); break;
+#define PQ_CASE(P) PQ_CASE2(P, 0) PQ_CASE2(P, 1) PQ_CASE2(P, 2)
     PQ_CASE(1) PQ_CASE(2) PQ_CASE(4) PQ_CASE(8) PQ_CASE(16) PQ_CASE(32)
 #undef PQ_CASE
+#undef PQ_CASE2
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

@@ -211,3 +211,38 @@ def test_reduce_outputs_and_extents(ctx, M, N, K):
         A, B = rand(rng, (M, K), ctx.np_dtype), rand(rng, (K, N), ctx.np_dtype)
         ia, ib = [-1, 1], [1, -2]
     check(ctx, A, ia, B, ib, run(ctx, A, ia, B, ib, _lib.KC_REDUCE))
+
+
+@pytest.mark.parametrize("K,N,k_first", [(1, 2, False), (2, 2, True), (2, 2, False), (4, 3, False), (7, 5, True),
+                                         (16, 4, False), (32, 8, False), (32, 1, True)])
+def test_stream_past_the_caches(ctx, K, N, k_first):
+    """Operand and result together over 384 MiB (loads and stores that pass
+    the caches), every K table size, lanes along and across the operand's
+    lines, an odd number of open elements."""
+    es = ctx.np_dtype.itemsize
+    M = (400 << 20) // es // (K + N) | 1
+    rng = np.random.default_rng(K * 10 + N)
+
+    def uniform(*shape):
+        r = rng.random(shape + (2,), dtype=np.float64 if es == 16 else np.float32)
+        r -= 0.5
+        return r.view(ctx.np_dtype)[..., 0]
+
+    # column-major tensors: numpy's row-major shapes reversed
+    X, Y = uniform(*((M, K) if k_first else (K, M))), uniform(N, K)
+    hx, hy = ctx.upload(X.T), ctx.upload(Y.T)
+    ctx.set_kernel_override(_lib.KC_STREAM)
+    try:
+        hz = ctx.contract(hx, [1, -1] if k_first else [-1, 1], hy, [1, -2])
+    finally:
+        ctx.set_kernel_override(-1)
+    got = ctx.download(hz).T                                   # [N, M]
+    for h in (hx, hy, hz):
+        ctx.free(h)
+    eps = 2.0 ** -53 if es == 16 else 2.0 ** -24
+    y = Y.astype(np.complex128)
+    for m in range(0, M, 1 << 20):
+        x = X[m:m + (1 << 20)].T if k_first else X[:, m:m + (1 << 20)]
+        x = x.astype(np.complex128)
+        bound = (np.abs(y) @ np.abs(x)) * (2 * K + 4) * eps
+        assert np.all(np.abs(got[:, m:m + (1 << 20)] - y @ x) <= bound)
