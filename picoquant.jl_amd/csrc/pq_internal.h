@@ -2,6 +2,8 @@
 // the kernel launchers.
 #pragma once
 #include "pq_common.h"
+
+#include <vector>
 #include "../../include/pq_hip.h"
 #include <string>
 
@@ -58,18 +60,18 @@ struct GemmArgs {
 
 // One problem of a grouped launch of small contractions (PQ_KC_BATCHED):
 // many independent steps of one dependency level in a single kernel launch,
-// one problem per grid row.  Pointers are for slice group 0; hA/hB/hC add
+// each on a run of workgroups of its own.  Pointers are for slice group 0; hA/hB/hC add
 // the leaf offset of each slice-group bit (group index passed at launch).
 #define PQ_MAX_HIGH_BITS 24
 struct MultiDesc {
   const void* A;
   const void* B;
   void* C;
-  Group M, N, K;      // as GenArgs
-  Batch L;            // batch entries of one slice group (grid z)
+  FDiv blocks;        // workgroups per batch entry
   int32_t conv;       // 1: element-type conversion of M.total elements A -> C (the other type)
-  int32_t c128;       // forest launches: the step computes in (conversions: converts from) complex128
   int32_t nhigh;
+  Group M, N, K;      // as GenArgs
+  Batch L;            // batch entries of one slice group
   int64_t hA[PQ_MAX_HIGH_BITS], hB[PQ_MAX_HIGH_BITS], hC[PQ_MAX_HIGH_BITS];
 };
 
@@ -77,8 +79,7 @@ struct MultiDesc {
 // decodes each offset in the loop)
 #define PQ_MULTI_KMAX 64
 template <typename C>
-hipError_t launch_multi(const MultiDesc* descs, int n, unsigned blocks_x, unsigned batch, int64_t group,
-                        hipStream_t s);
+hipError_t launch_multi(const MultiDesc* descs, const std::vector<uint32_t>& wgs, int64_t group, hipStream_t s);
 
 // Independent trees of small unbatched steps in one launch (k_forest), one
 // workgroup per tree, run level by level with a barrier between levels.

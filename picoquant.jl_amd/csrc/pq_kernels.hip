@@ -393,16 +393,34 @@ __global__ __launch_bounds__(256) void k_copy_bits(const C* __restrict__ In, C* 
 }
 
 // ----------------------------------------------------------------- k_multi
-// Grouped small contractions: problem blockIdx.y, batch entry blockIdx.z,
-// one lane per output element (grid-stride over blockIdx.x), loop over K;
-// a problem may instead be a small element-type conversion.
-template <typename C>
-__global__ __launch_bounds__(256) void k_multi(const MultiDesc* __restrict__ descs, int64_t group) {
-  const MultiDesc& d = descs[blockIdx.y];
+// Grouped small contractions: one lane per output element (strided over the
+// problem's workgroups of one batch entry), loop over K; a problem may
+// instead be a small element-type conversion.  Every problem has just the
+// workgroups it needs, found by comparing with the first one of each: a grid
+// of (most workgroups) x problems x (most batch entries) started 40960 of
+// them for some 700 with work where a wide and a batched problem met (25 us,
+// half a nanosecond for an empty one; 7 us now).  NP: 16 problems at most, or
+// 64 (a table for 64 alone cost every launch half a microsecond).
+template <int NP>
+struct MultiFirst {
+  uint32_t at[NP];   // past the last problem: none
+};
+template <typename C, int NP>
+__global__ __launch_bounds__(256) void k_multi(const MultiDesc* __restrict__ descs, MultiFirst<NP> first,
+                                               int64_t group) {
+  int p = 0;
+  uint32_t start = 0;
+#pragma unroll
+  for (int i = 1; i < NP; ++i) {
+    p = blockIdx.x >= first.at[i] ? i : p;
+    start = blockIdx.x >= first.at[i] ? first.at[i] : start;
+  }
+  const MultiDesc& d = descs[p];
   PQ_TOUCH(d.M, d.N, d.K, d.L);
-  if (blockIdx.z >= d.L.total) return;
+  const uint32_t entry = fdiv_q(blockIdx.x - start, d.blocks);
+  const uint32_t block = blockIdx.x - start - entry * d.blocks.d;
   int64_t oa, ob, oc;
-  batch_offsets(d.L, blockIdx.z, oa, ob, oc);
+  batch_offsets(d.L, entry, oa, ob, oc);
   for (int j = 0; j < d.nhigh; ++j)
     if ((group >> j) & 1) {
       oa += d.hA[j];
@@ -414,7 +432,7 @@ __global__ __launch_bounds__(256) void k_multi(const MultiDesc* __restrict__ des
     typedef typename std::conditional<sizeof(C) == 16, c64, c128>::type D;
     const C* A = reinterpret_cast<const C*>(d.A) + oa;
     D* Out = reinterpret_cast<D*>(d.C) + oc;
-    for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < d.M.total; t += gridDim.x * blockDim.x) {
+    for (uint32_t t = block * blockDim.x + threadIdx.x; t < d.M.total; t += d.blocks.d * blockDim.x) {
       const C v = A[t];
       D w;
       w.x = (decltype(w.x))v.x;
@@ -441,7 +459,7 @@ __global__ __launch_bounds__(256) void k_multi(const MultiDesc* __restrict__ des
     }
     __syncthreads();
   }
-  for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < total; t += gridDim.x * blockDim.x) {
+  for (uint32_t t = block * blockDim.x + threadIdx.x; t < total; t += d.blocks.d * blockDim.x) {
     uint32_t m = t % Mt, n = t / Mt;
     int32_t pa, pc1, pb, pc2;
     group_offsets(d.M, m, pa, pc1);
@@ -700,11 +718,26 @@ hipError_t launch_copy_bits(const C* In, C* Out, const CopyBitsArgs& a, hipStrea
   return hipGetLastError();
 }
 
+template <typename C, int NP>
+static void launch_problems(const MultiDesc* descs, const uint32_t* wgs, int n, int64_t group, hipStream_t s) {
+  MultiFirst<NP> first;
+  uint32_t total = 0;
+  for (int i = 0; i < NP; ++i) {
+    first.at[i] = i < n ? total : UINT32_MAX;
+    if (i < n) total += wgs[i];
+  }
+  hipLaunchKernelGGL((k_multi<C, NP>), dim3(total), dim3(256), 0, s, descs, first, group);
+}
+
 template <typename C>
-hipError_t launch_multi(const MultiDesc* descs, int n, unsigned blocks_x, unsigned batch, int64_t group,
-                        hipStream_t s) {
-  if (n < 1 || n > 65535 || batch < 1 || batch > 65535) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k_multi<C>), dim3(blocks_x, n, batch), dim3(256), 0, s, descs, group);
+hipError_t launch_multi(const MultiDesc* descs, const std::vector<uint32_t>& wgs, int64_t group, hipStream_t s) {
+  for (size_t p = 0; p < wgs.size(); p += 64) {
+    const int n = (int)std::min<size_t>(wgs.size() - p, 64);
+    if (n <= 16)
+      launch_problems<C, 16>(descs + p, wgs.data() + p, n, group, s);
+    else
+      launch_problems<C, 64>(descs + p, wgs.data() + p, n, group, s);
+  }
   return hipGetLastError();
 }
 
@@ -719,7 +752,7 @@ hipError_t launch_forest(const ForestStep* steps, const int4* items, const int2*
 }
 
 #define PQ_INST(C)                                                                                   \
-  template hipError_t launch_multi<C>(const MultiDesc*, int, unsigned, unsigned, int64_t, hipStream_t); \
+  template hipError_t launch_multi<C>(const MultiDesc*, const std::vector<uint32_t>&, int64_t, hipStream_t); \
   template hipError_t launch_stream<C>(const C*, const C*, C*, const StreamArgs&, hipStream_t);      \
   template hipError_t launch_generic<C>(const C*, const C*, C*, const GenArgs&, hipStream_t);        \
   template hipError_t launch_reduce<C>(const C*, const C*, C*, const GenArgs&, C*, int, hipStream_t); \

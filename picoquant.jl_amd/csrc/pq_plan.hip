@@ -173,7 +173,7 @@ struct Launch {
   std::vector<int> tree_start;  // forest: offset of each tree in steps, then steps.size()
   int desc_off = 0;
   int dtype = PQ_C128;
-  unsigned blocks_x = 1, batch = 1;
+  std::vector<uint32_t> wgs;    // grouped, not a forest: workgroups of each step
 };
 
 // Where a launch of a phase's sequence runs: its stream, the launches of the
@@ -784,10 +784,8 @@ int run_program(pq_ctx* c, pq_plan* p, bool profile_steps) {
                           c->stream);
       else
         e = (L.dtype == PQ_C128)
-                ? launch_multi<c128>(p->descs + L.desc_off, (int)L.steps.size(), L.blocks_x, L.batch, group,
-                                     c->stream)
-                : launch_multi<c64>(p->descs + L.desc_off, (int)L.steps.size(), L.blocks_x, L.batch, group,
-                                    c->stream);
+                ? launch_multi<c128>(p->descs + L.desc_off, L.wgs, group, c->stream)
+                : launch_multi<c64>(p->descs + L.desc_off, L.wgs, group, c->stream);
     }
     if (profile_steps) {
       hipEventRecord(p->ev[2 * L.steps[0] + 1], c->stream);
@@ -1158,7 +1156,9 @@ int create_plan(pq_ctx* c, const pq_plan_desc* d, int out_in_group, pq_plan** ou
     return st.kind == 1 && p->slots[st.a].dtype == PQ_C128 && p->slots[st.c].dtype == PQ_C64 &&
            conv_elems(st) <= 65536;
   };
-  // Grouped: contractions of at most 2^17 outputs and K <= PQ_MULTI_KMAX,
+  // Grouped: contractions of at most 2^17 outputs (all batch entries
+  // together: 64 entries of 2^14 took 25 us in a group, 10 alone) and K <=
+  // PQ_MULTI_KMAX,
   // whatever kernel they would run alone (small GEMMs too: two or more of
   // them per level share one launch instead of one launch each; on the 6x6
   // depth-14 plan 49 -> 36 launches and 1.40 -> 1.33 ms; at 2^18 / 2^19
@@ -1168,7 +1168,7 @@ int create_plan(pq_ctx* c, const pq_plan_desc* d, int out_in_group, pq_plan** ou
     return (st.kind == 0 &&
             (st.spec.kc == PQ_KC_STREAM || st.spec.kc == PQ_KC_GENERIC ||
              (st.spec.kc == PQ_KC_GEMM && st.spec.splitk <= 1)) &&
-            st.spec.Mt * st.spec.Nt <= (1u << 17) && st.spec.Kt <= PQ_MULTI_KMAX) ||
+            st.spec.Mt * st.spec.Nt * st.spec.L.total <= (1u << 17) && st.spec.Kt <= PQ_MULTI_KMAX) ||
            small_conv(st);
   };
   auto build_seq = [&](const std::vector<int>& order, std::vector<Launch>& seq) {
@@ -1349,13 +1349,11 @@ int create_plan(pq_ctx* c, const pq_plan_desc* d, int out_in_group, pq_plan** ou
     for (Launch& L : *seq) {
       if (!L.grouped || L.forest) continue;
       L.desc_off = (int)hd.size();
-      uint64_t maxw = 1;
-      unsigned maxb = 1;
       for (int i : L.steps) {
         const PStep& st = p->steps[i];
         MultiDesc m;
         memset(&m, 0, sizeof(m));
-        m.c128 = p->slots[st.a].dtype == PQ_C128 ? 1 : 0;
+        uint64_t work;
         m.A = slot_ptr(c, p, st.a, 0);
         m.B = slot_ptr(c, p, st.b, 0);
         m.C = slot_ptr(c, p, st.c, 0);
@@ -1368,15 +1366,14 @@ int create_plan(pq_ctx* c, const pq_plan_desc* d, int out_in_group, pq_plan** ou
             return fail(c, PQ_ERR_UNSUPPORTED, "grouped conversion too large");
           }
           m.L = single_batch();
-          maxw = std::max<uint64_t>(maxw, (uint64_t)n);
+          work = (uint64_t)n;
         } else {
           if (!fill_group(m.M, st.spec.M) || !fill_group(m.N, st.spec.N) || !fill_group(m.K, st.spec.K)) {
             free_plan(c, p);
             return fail(c, PQ_ERR_UNSUPPORTED, "too many modes in a grouped step");
           }
           m.L = st.spec.L;
-          maxw = std::max<uint64_t>(maxw, st.spec.Mt * st.spec.Nt);
-          maxb = std::max<unsigned>(maxb, st.spec.L.total);
+          work = st.spec.Mt * st.spec.Nt;
         }
         m.nhigh = st.phase2 ? d->n_sliced - group_bits : 0;
         for (int j = 0; j < m.nhigh; ++j) {
@@ -1386,13 +1383,13 @@ int create_plan(pq_ctx* c, const pq_plan_desc* d, int out_in_group, pq_plan** ou
           // a conversion's output keeps the same sliced bonds as its input
           m.hC[j] = st.kind == 1 ? p->slots[st.c].slice_stride[bit] : 0;
         }
+        // about one output per lane: a grouped problem's outputs are
+        // latency-bound chains of K loads (capped at 64 workgroups, a problem
+        // of 2^17 outputs took 8 per lane: 21-23 us against 10.5-11 us)
+        m.blocks = make_fdiv((uint32_t)std::min<uint64_t>((work + 255) / 256, 512));
+        L.wgs.push_back(m.blocks.d * m.L.total);
         hd.push_back(m);
       }
-      // about one output per lane: a grouped problem's outputs are
-      // latency-bound chains of K loads (capped at 64 workgroups, a problem
-      // of 2^17 outputs took 8 per lane: 21-23 us against 10.5-11 us)
-      L.blocks_x = (unsigned)std::min<uint64_t>((maxw + 255) / 256, 512);
-      L.batch = maxb;
     }
   }
   if (!hd.empty()) {

@@ -281,3 +281,48 @@ def test_concurrent_schedule_matches_one_stream(golden_dir, case):
     if case == "grid5x5_sliced":
         got = out[4].reshape(-1, order="F")
     assert np.linalg.norm(got - want) / np.linalg.norm(want) < tol
+
+
+@pytest.mark.parametrize("pairs", [2, 8, 9, 64, 65, 70])
+def test_levels_of_many_small_products(dtype, pairs):
+    """One dependency level of `pairs` independent small products (one
+    grouped launch up to 64, several past that), of 2048 outputs and more
+    each and of different sizes, so that each takes a run of workgroups of
+    its own; then the product of all of them."""
+    from picoquant_hip.network import Edge, Node
+    rng = np.random.default_rng(pairs)
+    tn = P.TensorNetworkCircuit.create(1, P.HIPBackend(dtype))
+    tn.edges.clear()
+    tn.input_qubits, tn.output_qubits = [], []
+    dims = [33 + 16 * (i % 4) for i in range(pairs + 1)]
+    dims[1::2] = [63 + i % 5 for i in range(len(dims[1::2]))]
+    want, mats = np.eye(dims[0]), []
+    for i in range(pairs):
+        k = 1 + i % 3
+        for sh in ((dims[i], k), (k, dims[i + 1])):
+            # one phase per factor: nothing cancels, so errors stay relative
+            mats.append((rng.uniform(0.5, 1, sh) / sh[1] * np.exp(1j * len(mats))).astype(dtype))
+    labels = [f"e{i}" for i in range(2 * pairs + 1)]
+    for i, m in enumerate(mats):
+        lab = f"node_{i + 1}"
+        tn.nodes[lab] = Node([labels[i], labels[i + 1]], list(m.shape), lab)
+        tn.backend.save_tensor_data(lab, m)
+        want = want @ m.astype(np.complex128)
+    for i, e in enumerate(labels):
+        tn.edges[e] = Edge(f"node_{i}" if i else None, f"node_{i + 1}" if i < 2 * pairs else None)
+    tn.counters["node"] = 2 * pairs
+    plan = [(f"node_{2 * i + 1}", f"node_{2 * i + 2}") for i in range(pairs)]
+    last = f"node_{2 * pairs + 1}"
+    for i in range(1, pairs):
+        plan.append((last, f"node_{2 * pairs + 1 + i}"))
+        last = f"node_{2 * pairs + len(plan)}"
+    p = compile_plan(tn, plan, out_order=[labels[0], labels[-1]])
+    p.execute(use_graph=False)
+    got = p.result()
+    p.execute(use_graph=True)
+    assert np.array_equal(p.result(), got)
+    p.close()
+    # each summed element and each factor rounds once; complex products up to 2 sqrt(2)
+    terms = sum(m.shape[1] + 2 for m in mats)
+    eps = 2.0 ** -53 if dtype == np.complex128 else 2.0 ** -24
+    assert np.all(np.abs(got - want) <= 4 * terms * eps * np.abs(want))
