@@ -109,7 +109,8 @@ struct ForestCopy {
 };
 // A tree's LDS: its step records (32-bit words, padded to 8 bytes), its K
 // offsets, then (16-byte aligned) its data area.  Per-lane leaf copies:
-#define PQ_FOREST_COPY_PER_LANE 8
+#define PQ_FOREST_LANES 1024
+#define PQ_FOREST_COPY_PER_LANE 2
 // lds_bytes: LDS of the largest tree (0: the kernel reads records and K
 // offsets from global memory and keeps every operand there), at most
 // PQ_FOREST_LDS_BYTES

@@ -537,8 +537,12 @@ __device__ __forceinline__ void forest_item(const ForestStep& f, const int4& it,
 // reads, live in the LDS data area after them (leaves copied in at the
 // start), so only the other leaves and the tree's root result go through
 // global memory.
+// Bound: the levels' latency, one after another.  1024 lanes, since a level
+// of a few thousand outputs left 256 with several in turn: 24 us instead of
+// 38 for 44 trees of 16 levels, 33 instead of 44 for 69 (512 lanes: a
+// microsecond longer).
 template <bool LDS>
-__global__ __launch_bounds__(256) void k_forest(const ForestStep* __restrict__ fs, const int4* __restrict__ items,
+__global__ __launch_bounds__(PQ_FOREST_LANES) void k_forest(const ForestStep* __restrict__ fs, const int4* __restrict__ items,
                                                 const int2* __restrict__ ktab,
                                                 const ForestCopy* __restrict__ copies,
                                                 const int32_t* __restrict__ lv) {
@@ -558,7 +562,7 @@ __global__ __launch_bounds__(256) void k_forest(const ForestStep* __restrict__ f
     int32_t cd[PQ_FOREST_COPY_PER_LANE];
 #pragma unroll
     for (int j = 0; j < PQ_FOREST_COPY_PER_LANE; ++j) {
-      const int32_t e = tid + 256 * j;
+      const int32_t e = tid + PQ_FOREST_LANES * j;
       if (e < nc) {
         const ForestCopy cp = copies[c0 + e];
         cv[j] = *reinterpret_cast<const float2*>(cp.src);
@@ -573,7 +577,7 @@ __global__ __launch_bounds__(256) void k_forest(const ForestStep* __restrict__ f
     dat = reinterpret_cast<char*>(fsm) + (((size_t)kw * 4 + (size_t)nkt * 8 + 15) & ~(size_t)15);
 #pragma unroll
     for (int j = 0; j < PQ_FOREST_COPY_PER_LANE; ++j)
-      if (tid + 256 * j < nc) *reinterpret_cast<float2*>(dat + cd[j]) = cv[j];
+      if (tid + PQ_FOREST_LANES * j < nc) *reinterpret_cast<float2*>(dat + cd[j]) = cv[j];
     __syncthreads();
     F = reinterpret_cast<const ForestStep*>(fsm);
     KT = kd;
@@ -745,9 +749,9 @@ hipError_t launch_forest(const ForestStep* steps, const int4* items, const int2*
                          const int32_t* lv, int ntrees, size_t lds_bytes, hipStream_t s) {
   if (ntrees < 1 || ntrees > (1 << 24) || lds_bytes > PQ_FOREST_LDS_BYTES) return hipErrorInvalidValue;
   if (lds_bytes > 0)
-    hipLaunchKernelGGL(k_forest<true>, dim3(ntrees), dim3(256), lds_bytes, s, steps, items, ktab, copies, lv);
+    hipLaunchKernelGGL(k_forest<true>, dim3(ntrees), dim3(PQ_FOREST_LANES), lds_bytes, s, steps, items, ktab, copies, lv);
   else
-    hipLaunchKernelGGL(k_forest<false>, dim3(ntrees), dim3(256), 0, s, steps, items, ktab, copies, lv);
+    hipLaunchKernelGGL(k_forest<false>, dim3(ntrees), dim3(PQ_FOREST_LANES), 0, s, steps, items, ktab, copies, lv);
   return hipGetLastError();
 }
 

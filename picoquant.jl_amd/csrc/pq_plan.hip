@@ -1533,7 +1533,7 @@ int create_plan(pq_ctx* c, const pq_plan_desc* d, int out_in_group, pq_plan** ou
         };
         const int32_t c0 = (int32_t)copies.size();
         int64_t pieces = 0, high = 0;
-        const int64_t max_pieces = 256 * PQ_FOREST_COPY_PER_LANE;
+        const int64_t max_pieces = PQ_FOREST_LANES * PQ_FOREST_COPY_PER_LANE;
         for (int r = fs0; r < fs0 + nfs; ++r) {
           const PStep& st = p->steps[fstep[r]];
           for (int o = 0; o < (st.kind == 1 ? 1 : 2); ++o) {
