@@ -342,8 +342,11 @@ __global__ __launch_bounds__(PQ_PUT_WORDS) void k_put(uint32_t* __restrict__ dst
 // low 8 bits once, the rest uniform, where k_copy decodes every element
 // through all modes and reads one element of each line it touches.
 // Bound: HBM (2^24 complex64 elements in a random axis order: 48 us = 5.5
-// TB/s, 107 us by k_copy, whose time is its per-element decode).
-template <typename C>
+// TB/s, 107 us by k_copy, whose time is its per-element decode).  NT: In and
+// Out are together well over the 256 MB last-level cache and Out passes it
+// (2^24 complex128, three tensors in turn 109 -> 104 us and 107 -> 98, one
+// again and again 121 -> 80).
+template <typename C, bool NT>
 __global__ __launch_bounds__(256) void k_copy_bits(const C* __restrict__ In, C* __restrict__ Out, CopyBitsArgs a) {
   constexpr int NB = CB_BITS(sizeof(C)), PER = 1 << (NB - 8);
   __shared__ C tile[1 << NB];
@@ -388,7 +391,7 @@ __global__ __launch_bounds__(256) void k_copy_bits(const C* __restrict__ In, C* 
         o += a.os[b];
         t ^= a.ol[b];
       }
-    out[o] = tile[t];
+    store_one<NT>(out + o, tile[t]);
   }
 }
 
@@ -718,7 +721,11 @@ hipError_t launch_put(void* dst, const void* host, int n, hipStream_t s) {
 
 template <typename C>
 hipError_t launch_copy_bits(const C* In, C* Out, const CopyBitsArgs& a, hipStream_t s) {
-  hipLaunchKernelGGL((k_copy_bits<C>), dim3(a.outer.total), dim3(256), 0, s, In, Out, a);
+  const dim3 grid(a.outer.total), block(256);
+  if (2.0 * a.outer.total * (1 << CB_BITS(sizeof(C))) * sizeof(C) > 384.0 * (1 << 20))
+    hipLaunchKernelGGL((k_copy_bits<C, true>), grid, block, 0, s, In, Out, a);
+  else
+    hipLaunchKernelGGL((k_copy_bits<C, false>), grid, block, 0, s, In, Out, a);
   return hipGetLastError();
 }
 

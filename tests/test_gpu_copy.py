@@ -65,3 +65,10 @@ def test_sliced_views(ctx, axis):
     check(ctx, dims, perm, (where, 2, 2))
     other = axis if axis != where else axis + 1
     check(ctx, dims, perm, (other, 2, 2))
+
+
+def test_past_the_caches(ctx):
+    """Tensor and copy together over 384 MiB (stores that pass the caches),
+    an odd factor among the extents."""
+    dims = [2] * 22 + ([5] if ctx.np_dtype == np.complex128 else [2, 5])
+    check(ctx, dims, np.random.default_rng(len(dims)).permutation(len(dims)).tolist())
