@@ -2,7 +2,7 @@
 
 The drivers keep the reference's labels, layer order and rewiring; their
 work runs on the GPU through the backend verbs: contract_tensors
-(pq_contract) and decompose_tensor (pq_decompose, rocSOLVER's SVD with the
+(pq_contract) and decompose_tensor (pq_decompose, an SVD with the
 reference's threshold / max_rank rule for the bond dimension).
 """
 from __future__ import annotations
