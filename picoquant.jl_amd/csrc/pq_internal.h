@@ -146,9 +146,9 @@ int gemm_k_limit();
 bool gemm16_applicable(const GemmArgs& g);
 hipError_t launch_gemm16(const c64* A, const c64* B, c64* Out, const GemmArgs& a, hipStream_t s);
 
-// Number of partial blocks the split-K reduction uses for a K extent and a
-// number of batch entries.
-int reduce_blocks_for(uint32_t ktotal, uint32_t batch);
+// Number of partial blocks the split-K reduction uses for a K extent, a
+// number of batch entries and one of outputs per entry.
+int reduce_blocks_for(uint32_t ktotal, uint32_t batch, uint32_t outputs);
 
 // Fused chain of small complex64 operators on one large tensor (plan steps
 // of kind 2; the program format is documented with PQ_CHAIN_* in pq_hip.h).

@@ -152,8 +152,9 @@ __global__ __launch_bounds__(256) void k_generic(const C* __restrict__ A, const 
 // parts of its next 64 steps together (decoded per step on the scalar unit,
 // 23 modes held the loop at 68 us where the loads alone take 46).
 // Bound: HBM for long K (2^23 against 2^23 complex128: 180 us before, 53.5
-// now at 53 for the bytes), two launches for short (a call on 2^14 x 2^13
-// elements closed over 2^13: 39 us on 2 workgroups, 15 on 16).
+// now at 53 for the bytes), the launches for short (a call on 2^14 x 2^13
+// elements closed over 2^13: 39 us on 2 workgroups, 15 on 16; an overlap of
+// two 12-qubit states 14 us in two launches, 11 in one).
 template <typename C, int TM, int TN>
 __global__ __launch_bounds__(256) void k_reduce_partial(const C* __restrict__ A, const C* __restrict__ B,
                                                         C* __restrict__ partials, C* __restrict__ Out, GenArgs a) {
@@ -667,8 +668,12 @@ hipError_t launch_generic(const C* A, const C* B, C* Out, const GenArgs& a, hipS
   return hipGetLastError();
 }
 
-int reduce_blocks_for(uint32_t ktotal, uint32_t batch) {
-  // 4096 values of K per workgroup (16 per lane) and at most 2048 workgroups;
+int reduce_blocks_for(uint32_t ktotal, uint32_t batch, uint32_t outputs) {
+  // one workgroup, which needs no second launch, for up to 4096 values of K
+  // and 2^15 products (2 x 2 outputs over 4096: 6.3 us, 9.6 in eight parts;
+  // 16 over 2048 12.3 and 13.2, over 4096 16.2 and 13.1)
+  if (ktotal <= 4096 && (uint64_t)ktotal * outputs <= 1u << 15) return 1;
+  // 4096 values per workgroup (16 per lane) and at most 2048 workgroups;
   // fewer values, down to 512, while that keeps the device short of 2048
   const uint32_t least = ktotal / 4096, fill = std::min(ktotal / 512, 2048u / std::max(batch, 1u));
   return (int)std::min(std::max(std::max(least, fill), 1u), 2048u);

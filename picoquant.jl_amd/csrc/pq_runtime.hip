@@ -566,7 +566,8 @@ int prepare_contract(pq_ctx* c, const Tensor& A, int ra, const int32_t* ia, cons
 size_t step_scratch_bytes(const StepSpec& s, size_t esize) {
   if (s.kc == PQ_KC_GEMM && s.splitk > 1) return (size_t)s.splitk * s.Mt * s.Nt * esize;
   if (s.kc != PQ_KC_REDUCE) return 0;
-  return (size_t)reduce_blocks_for((uint32_t)s.Kt, s.L.total) * s.Mt * s.Nt * s.L.total * esize;
+  return (size_t)reduce_blocks_for((uint32_t)s.Kt, s.L.total, (uint32_t)(s.Mt * s.Nt)) * s.Mt * s.Nt * s.L.total *
+         esize;
 }
 
 template <typename C>
@@ -689,8 +690,8 @@ static int launch_typed(pq_ctx* c, const C* pa, const C* pb, C* pc, const StepSp
     ga.L = s.L;
     if (s.kc == PQ_KC_REDUCE) {
       ProfScope ps(c, PQ_KC_REDUCE, alg_bytes, alg_flops);
-      e = launch_reduce<C>(pa, pb, pc, ga, reinterpret_cast<C*>(scratch), reduce_blocks_for((uint32_t)s.Kt, s.L.total),
-                           c->stream);
+      e = launch_reduce<C>(pa, pb, pc, ga, reinterpret_cast<C*>(scratch),
+                           reduce_blocks_for((uint32_t)s.Kt, s.L.total, (uint32_t)(s.Mt * s.Nt)), c->stream);
     } else {
       ProfScope ps(c, PQ_KC_GENERIC, alg_bytes, alg_flops);
       e = launch_generic<C>(pa, pb, pc, ga, c->stream);
