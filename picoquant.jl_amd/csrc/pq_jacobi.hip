@@ -154,13 +154,15 @@ template <> struct Tol<double> {
   static constexpr double cos2 = 1e-30;    // rotate while |x^H y|^2 > cos2 |x|^2 |y|^2
   static constexpr double done = 1e-17;    // squared angle and cosine that one more sweep would square
   static constexpr double floor2 = 1e-20;  // columns below 1e-10 of the whole are far under any cut-off
-  static constexpr double tiny = 1e-280;   // squares below this count as zero
+  static constexpr double zero2 = 1e-250;  // a column's squared norm that counts as zero (largest element 1)
+  static constexpr double small2 = 1e-34;  // an element whose square is this part of its column's counts as zero
 };
 template <> struct Tol<float> {
   static constexpr float cos2 = 9e-14f;
   static constexpr float done = 1e-8f;
   static constexpr float floor2 = 1e-12f;
-  static constexpr float tiny = 1e-34f;
+  static constexpr float zero2 = 1e-20f;
+  static constexpr float small2 = 1e-17f;
 };
 
 // Sum over the 8 lanes of a half row, in each of them.
@@ -370,31 +372,38 @@ __global__ __launch_bounds__(JAC_THREADS) void k_jacobi(JacArgs j, Ordering o) {
   };
   for (int k = 0; k < q; ++k) {
     C v[RP];
-    R n2 = 0;
+    R b2 = 0;                                       // squared norm below the diagonal
 #pragma unroll
     for (int t = 0; t < RP; ++t) {
       v[t] = A[k * PP + l + 16 * t];
-      if (l + 16 * t < k) v[t].x = v[t].y = 0;
-      n2 = fma(v[t].x, v[t].x, fma(v[t].y, v[t].y, n2));
+      if (l + 16 * t <= k) v[t].x = v[t].y = 0;
+      b2 = fma(v[t].x, v[t].x, fma(v[t].y, v[t].y, b2));
     }
     const C d = A[k * PP + k];
-    n2 = row_sum(n2);
+    b2 = row_sum(b2);
     const R d2 = fma(d.x, d.x, d.y * d.y);
-    const bool some = n2 > Tol<R>::tiny, ang = d2 > Tol<R>::tiny;
-    const R nx = some ? n2 * rsq_full(n2) : R(0), id = ang ? rsq_full(d2) : R(0);
-    C ph, v0;
-    ph.x = ang ? d.x * id : R(1);
-    ph.y = ang ? d.y * id : R(0);
-    v0.x = fma(ph.x, nx, d.x);
-    v0.y = fma(ph.y, nx, d.y);
-    const R f = some ? rcp_full(fma(nx, d2 * id, n2)) : R(0);
+    // H is unitary for any v, as f = 2 / |v|^2 of the very v it is applied
+    // with; that H maps the column onto the diagonal decides v.  A column
+    // that is zero below the diagonal (under any rounding of the matrix) is
+    // left alone; a diagonal element under the rounding of the rest counts
+    // as zero, so that its phase is never taken from a square that vanishes.
+    const bool some = !(b2 <= Tol<R>::zero2), ang = d2 > Tol<R>::small2 * b2;
+    const R n2 = b2 + d2, nx = n2 * rsq_full(n2), id = ang ? rsq_full(d2) : R(0);
+    C v0, rd;                                       // rd: the column's element of R
+    rd.x = ang ? d.x * id * nx : nx;
+    rd.y = ang ? d.y * id * nx : R(0);
+    v0.x = ang ? rd.x + d.x : nx;
+    v0.y = ang ? rd.y + d.y : R(0);
+    const R f = some ? R(2) * rcp_full(fma(v0.x, v0.x, fma(v0.y, v0.y, b2))) : R(0);
+    rd.x = some ? -rd.x : d.x;
+    rd.y = some ? -rd.y : d.y;
 #pragma unroll
     for (int t = 0; t < RP; ++t)
       if (l + 16 * t == k) v[t] = v0;
     reflect(v, f, k, true);
     if (grp == (k & (JAC_GROUPS - 1)) && l == 0) {
-      L[k * LR + k].x = -ph.x * nx;
-      L[k * LR + k].y = ph.y * nx;
+      L[k * LR + k].x = rd.x;
+      L[k * LR + k].y = -rd.y;
       v0s[k] = v0;
       fs[k] = f;
     }

@@ -120,3 +120,25 @@ def test_strided_tensor(ctx):
     assert np.array_equal(ctx.download(h), T.astype(ctx.np_dtype))       # not consumed
     for x in (h, hp, hv, hb, hc):
         ctx.free(x)
+
+
+@pytest.mark.parametrize("wide", [False, True], ids=["tall", "wide"])
+@pytest.mark.parametrize("m,n,col", [(4, 2, 0), (4, 3, 0), (4, 4, 1), (6, 5, 2), (33, 20, 7)])
+def test_nearly_zero_columns(ctx, m, n, col, wide):
+    """A column of the size of a rounding error (cos(pi/2) = 6e-17 in a gate)
+    in front of columns of ordinary size, over the scales where its square
+    leaves the type's range, its diagonal element as large as the rest,
+    smaller or zero.  With `col` > 0 the columns before it only touch the
+    rows above, so the reflections before it leave it as it is."""
+    rng = np.random.default_rng(10 * m + n)
+    lo, hi = (1e-21, 1e-7) if ctx.np_dtype == np.complex64 else (1e-146, 1e-125)
+    for scale in np.geomspace(lo, hi, 57):
+        for diag in (1.0, 0.3, 1e-2, 1e-6, 0.0):
+            A = rnd(rng, m, n)
+            A[col:, :col] = 0
+            A[:, col] *= scale
+            A[:col, col] = 0
+            A[col, col] *= diag
+            A = A.astype(ctx.np_dtype).astype(np.complex128)
+            A = A.T if wide else A
+            check(ctx, A, *split(ctx, A))
