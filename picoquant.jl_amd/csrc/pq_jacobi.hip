@@ -154,6 +154,7 @@ template <> struct Tol<double> {
   static constexpr double cos2 = 1e-30;    // rotate while |x^H y|^2 > cos2 |x|^2 |y|^2
   static constexpr double done = 1e-17;    // squared angle and cosine that one more sweep would square
   static constexpr double floor2 = 1e-20;  // columns below 1e-10 of the whole are far under any cut-off
+  static constexpr double least = 2.3e-308;   // under this a square is subnormal or zero
   static constexpr double zero2 = 1e-250;  // a column's squared norm that counts as zero (largest element 1)
   static constexpr double small2 = 1e-34;  // an element whose square is this part of its column's counts as zero
 };
@@ -161,6 +162,7 @@ template <> struct Tol<float> {
   static constexpr float cos2 = 9e-14f;
   static constexpr float done = 1e-8f;
   static constexpr float floor2 = 1e-12f;
+  static constexpr float least = 1.2e-38f;
   static constexpr float zero2 = 1e-20f;
   static constexpr float small2 = 1e-17f;
 };
@@ -232,9 +234,11 @@ __device__ __forceinline__ void rotate2(C (&x)[4][LRP], R (&n)[4], R fl, bool& b
   const R nu = hi ? n[U2] : n[U], nw = hi ? n[W2] : n[W];
   const R g2 = fma(gr, gr, gi * gi);
   const R nn = fmax(nu, fl) * fmax(nw, fl);
-  const bool rot = g2 > Tol<R>::cos2 * nn;
-  // the angle from raw estimates: any w = s / c gives a unitary rotation, as
-  // c is computed from w itself
+  // (a subnormal g2, which two columns far under the floor can have in
+  // float, has no 1 / sqrt: the instruction returns infinity for it)
+  const bool rot = g2 > fmax(Tol<R>::cos2 * nn, Tol<R>::least);
+  // the angle from raw estimates: any finite w = s / c gives a unitary
+  // rotation, as c is computed from w itself
   const R ig = rsq_raw(g2);
   const R ze = R(0.5) * (nw - nu) * ig;
   const R ta = rcp_raw(fabs(ze) + sqrt_raw(fma(ze, ze, R(1))));

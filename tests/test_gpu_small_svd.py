@@ -142,3 +142,20 @@ def test_nearly_zero_columns(ctx, m, n, col, wide):
             A = A.astype(ctx.np_dtype).astype(np.complex128)
             A = A.T if wide else A
             check(ctx, A, *split(ctx, A))
+
+
+@pytest.mark.parametrize("g", [7.7e-20, 8.2e-20, 9e-20, 1e-19, 1.07e-19, 1.2e-19, 5e-19])
+def test_columns_with_a_subnormal_inner_product(ctx, g):
+    """Two columns far below the cut-off whose inner product's square is
+    subnormal in complex64: one singular value is left, and the split stays
+    on the kernel -- the library's path starts with a copy of the tensor,
+    which the profile counts."""
+    b = np.sqrt(g)
+    A = np.array([[0.5, 0, 0], [0, b, b], [0, 0, b]], dtype=complex)
+    ctx.profile_enable(True)
+    B, C, chi = split(ctx, A)
+    copies = ctx.profile_read(_lib.KC_COPY)["launches"]
+    ctx.profile_enable(False)
+    assert copies == 0
+    assert chi == 1
+    assert np.allclose(B @ C, np.diag([0.5, 0, 0]), rtol=0, atol=1e-7)
