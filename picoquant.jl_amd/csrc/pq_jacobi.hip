@@ -396,8 +396,8 @@ __global__ __launch_bounds__(JAC_THREADS) void k_jacobi(JacArgs j, Ordering o) {
     C v0, rd;                                       // rd: the column's element of R
     rd.x = ang ? d.x * id * nx : nx;
     rd.y = ang ? d.y * id * nx : R(0);
-    v0.x = ang ? rd.x + d.x : nx;
-    v0.y = ang ? rd.y + d.y : R(0);
+    v0.x = !some ? R(0) : (ang ? rd.x + d.x : nx);  // (nx is NaN for a zero column)
+    v0.y = some && ang ? rd.y + d.y : R(0);
     const R f = some ? R(2) * rcp_full(fma(v0.x, v0.x, fma(v0.y, v0.y, b2))) : R(0);
     rd.x = some ? -rd.x : d.x;
     rd.y = some ? -rd.y : d.y;

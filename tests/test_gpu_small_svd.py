@@ -159,3 +159,25 @@ def test_columns_with_a_subnormal_inner_product(ctx, g):
     assert copies == 0
     assert chi == 1
     assert np.allclose(B @ C, np.diag([0.5, 0, 0]), rtol=0, atol=1e-7)
+
+
+@pytest.mark.parametrize("wide", [False, True], ids=["tall", "wide"])
+@pytest.mark.parametrize("m,n,zero", [(4, 4, [3]), (4, 4, [0]), (6, 4, [1, 2]), (16, 9, [0, 8]), (40, 33, [5, 32]),
+                                      (5, 1, []), (1, 1, [])])
+def test_zero_columns(ctx, m, n, zero, wide):
+    """Columns that are zero, or zero below the diagonal: split by the
+    kernel itself (the library's path starts with a copy)."""
+    rng = np.random.default_rng(m + n)
+    for tail in (False, True):
+        A = rnd(rng, m, n)
+        A[:, zero] = 0
+        if tail:
+            A = np.triu(A)
+        A = A.astype(ctx.np_dtype).astype(np.complex128)
+        A = A.T if wide else A
+        ctx.profile_enable(True)
+        got = split(ctx, A)
+        copies = ctx.profile_read(_lib.KC_COPY)["launches"]
+        ctx.profile_enable(False)
+        assert copies == 0
+        check(ctx, A, *got)
