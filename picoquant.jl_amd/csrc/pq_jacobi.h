@@ -11,6 +11,7 @@
 
 struct JacMeta {
   double root[JAC_MAX_Q];   // sqrt of column c's singular value
+  double rest[JAC_MAX_Q];   // ... and what its rounding left
   int32_t pos[JAC_MAX_Q];   // its place in descending order
   int32_t chi, lines;
 };

@@ -2,11 +2,15 @@
 // two launches: Householder QR and one-sided Jacobi in one workgroup's LDS,
 // then the left rotations replayed on many.  For pq_decompose's matrices --
 // two MPS sites merged over a bond of at most 32 -- the library SVD is some
-// 50 to 100 dependent launches (197 us for 2 x 2, 0.77 ms for 16 x 16, 3.2 ms
-// for 64 x 64 complex128, calls included); this takes 28 us, 95 us and 0.67
-// ms.  Its errors on random matrices are 1 to 4 times the library's (recon-
-// structions 3.7e-15 against 2.5e-15 at 64 x 64) and far below them on graded
-// ones (spectra over ten decades: 3e-15 against 2e-8).
+// 50 to 100 dependent launches (140 to 190 us for 2 x 2, 0.67 ms for 16 x 16,
+// 2.4 ms for 64 x 64 complex128, calls included); this takes 30 us, 99 us and
+// 0.70 ms.  Errors, as |X - B C| / |X| over random matrices (library in
+// brackets): complex128 7.1e-16 (1.4e-15) at 16 x 16 and 1.5e-15 (2.0e-15) at
+// 64 x 64, complex64 3.7e-7 (9.1e-7) and 7.3e-7 (1.1e-6); equal at 2 x 2, and
+// far smaller on graded spectra (six decades, 16 x 16: 6.9e-16 against
+// 8.6e-12).  Singular values and orthogonality likewise.  Only the smallest
+// singular values of graded matrices of up to 8 columns are less exact, 0.3 of
+// an ulp of the largest against 0.1.
 //
 //   X (m x n, or its conjugate transpose when m < n) = A (p x q), p >= q
 //   A = Q R (Householder);  L = R^H
@@ -26,10 +30,11 @@
 // cosets of GF(4)* in GF(64)* and GF(16)*; odd powers of two have no such
 // partition and keep a few single r's).  16 lanes hold a group's rows, so
 // every inner product is a sum over a DPP row.
-// Bound: instruction issue of one wave per SIMD of one CU -- 575 us of the 64
+// Bound: instruction issue of one wave per SIMD of one CU -- 612 us of the 64
 // x 64 call are the one workgroup (8 sweeps of 21 lines, a fifth of it QR),
-// 67 the replay.  The round-robin of dependent rounds leaves nothing for
-// other CUs.
+// 73 the replay.  The round-robin of dependent rounds leaves nothing for
+// other CUs.  One rounding per element and rotation (turn, times) costs 6 % of
+// that over c x - s y with rounded factors and halves the errors.
 #include "pq_jacobi.h"
 
 #include <cmath>
@@ -45,7 +50,7 @@ namespace {
 // they would go through the vector memory counter and wait for the log's
 // stores.
 #define JAC_MAX_LINES 21
-#define JAC_LOG 18            // log entries of a group and line: (Re s, Im s, c) of six rotations
+#define JAC_LOG 18            // log entries of a group and line: (Re s, Im s, 1 - c) of six rotations
 struct Ordering {
   uint32_t line[JAC_MAX_LINES];
   int nline;
@@ -130,11 +135,13 @@ __device__ __forceinline__ double rcp_raw(double x) { return __builtin_amdgcn_rc
 __device__ __forceinline__ float rcp_raw(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ __forceinline__ double sqrt_raw(double x) { return __builtin_amdgcn_sqrt(x); }
 __device__ __forceinline__ float sqrt_raw(float x) { return __builtin_amdgcn_sqrtf(x); }
-// 1 / sqrt(x) to within half an ulp or so (x > 0, its square root normal): a
-// Newton step on the estimate, then one on the exact residual.  Every
-// rotation scales its columns by this value's error, hundreds of times over:
-// plain Newton steps left a bias that cost a 64-column matrix 2e-14 in its
-// singular values (4e-15 with the exact residual).
+// 1 / sqrt(x) (x > 0, its square root normal): to a few ulp, and to within
+// half an ulp or so by one more step on the exact residual.
+__device__ __forceinline__ float rsq_near(float x) { return rsq_raw(x); }
+__device__ __forceinline__ double rsq_near(double x) {
+  const double y = rsq_raw(x);
+  return fma(y, 0.5 * fma(-x * y, y, 1.0), y);
+}
 template <typename R>
 __device__ __forceinline__ R rsq_full(R x) {
   R y = rsq_raw(x);
@@ -175,15 +182,22 @@ __device__ __forceinline__ R half_sum(R v) {
   v += dpp_mov<0xb1>(v);   // quad_perm 1, 0, 3, 2
   return v;
 }
-// x' = c x - s y,  y' = c y + conj(s) x
+// x' = c x - s y,  y' = c y + conj(s) x  with c = 1 - k: the change is summed
+// first and x added last, so an element is rounded once at its own size
+// whatever the number of terms (as c x - s y, three times: the errors of 64
+// columns, eight sweeps of 63 rotations each, were 2 times the present ones).
 template <typename R, typename C>
-__device__ __forceinline__ void turn(C& x, C& y, R sr, R si, R c) {
+__device__ __forceinline__ void turn(C& x, C& y, R sr, R si, R k) {
   const C a = x, b = y;
-  x.x = fma(-sr, b.x, fma(si, b.y, c * a.x));
-  x.y = fma(-sr, b.y, fma(-si, b.x, c * a.y));
-  y.x = fma(sr, a.x, fma(si, a.y, c * b.x));
-  y.y = fma(sr, a.y, fma(-si, a.x, c * b.y));
+  x.x = a.x - fma(sr, b.x, fma(-si, b.y, k * a.x));
+  x.y = a.y - fma(sr, b.y, fma(si, b.x, k * a.y));
+  y.x = b.x + fma(sr, a.x, fma(si, a.y, -k * b.x));
+  y.y = b.y + fma(sr, a.y, fma(-si, a.x, -k * b.y));
 }
+
+// v (h + l), rounded once: l is what rounding h left of a factor.
+__device__ __forceinline__ float times(float v, double h, double) { return (float)((double)v * h); }
+__device__ __forceinline__ double times(double v, double h, double l) { return fma(v, h, v * l); }
 
 // The four columns of group g on a line: c0 is the one with both pivot bits
 // clear.
@@ -206,7 +220,7 @@ __device__ __forceinline__ bool three_rounds(uint32_t line) { return (line >> 22
 // is the number of instructions: no branches, and the two pairs share the
 // sums and the angle -- lanes 0-7 of the row take the first pair, lanes 8-15
 // the second, and swap the results.  A pair that needs no rotation gets s =
-// 0, c = 1.
+// 0, c = 1 (k = 1 - c = 0).
 template <typename R, typename C, int LRP, int U, int W, int U2, int W2>
 __device__ __forceinline__ void rotate2(C (&x)[4][LRP], R (&n)[4], R fl, bool& big, R* e, int l) {
   R g[2][2];
@@ -237,32 +251,37 @@ __device__ __forceinline__ void rotate2(C (&x)[4][LRP], R (&n)[4], R fl, bool& b
   // (a subnormal g2, which two columns far under the floor can have in
   // float, has no 1 / sqrt: the instruction returns infinity for it)
   const bool rot = g2 > fmax(Tol<R>::cos2 * nn, Tol<R>::least);
-  // the angle from raw estimates: any finite w = s / c gives a unitary
-  // rotation, as c is computed from w itself
+  // the angle from raw estimates: any finite s of at most sqrt(1/2) gives a
+  // unitary rotation, as k = 1 - c is computed from s itself
   const R ig = rsq_raw(g2);
   const R ze = R(0.5) * (nw - nu) * ig;
   const R ta = rcp_raw(fabs(ze) + sqrt_raw(fma(ze, ze, R(1))));
   const R t = rot ? (ze < 0 ? -ta : ta) : R(0);
   const R ti = rot ? t * ig : R(0);
   const R wr = ti * gr, wi = -ti * gi;
-  const R c = rsq_full(fma(wr, wr, fma(wi, wi, R(1))));
-  const R sr = c * wr, si = c * wi, d = ti * g2;
+  const R x2 = fma(wr, wr, fma(wi, wi, R(1))), c0 = rsq_near(x2);
+  const R sr = c0 * wr, si = c0 * wi, d = ti * g2;
+  // k (2 - k) = |s|^2: an estimate, then a Newton step on the residual.  Its
+  // error is far below an ulp of 1, so repeated rotations do not scale the
+  // columns.
+  const R s2 = fma(sr, sr, si * si), k0 = s2 * rcp_raw(R(1) + c0);
+  const R k = fma(fma(k0, k0, fma(R(-2), k0, s2)), R(0.5) * x2 * c0, k0);
   big = big || (rot && (g2 > Tol<R>::done * nn || t * t > Tol<R>::done));
   if ((l & 7) == 0) {
     R* q = e + 3 * (l >> 3);
     q[0] = sr;
     q[1] = si;
-    q[2] = c;
+    q[2] = k;
   }
-  const R osr = dpp_mov<0x128>(sr), osi = dpp_mov<0x128>(si), oc = dpp_mov<0x128>(c), od = dpp_mov<0x128>(d);
+  const R osr = dpp_mov<0x128>(sr), osi = dpp_mov<0x128>(si), ok = dpp_mov<0x128>(k), od = dpp_mov<0x128>(d);
   const R zr[2] = {hi ? osr : sr, hi ? sr : osr}, zi[2] = {hi ? osi : si, hi ? si : osi},
-          zc[2] = {hi ? oc : c, hi ? c : oc}, zd[2] = {hi ? od : d, hi ? d : od};
+          zk[2] = {hi ? ok : k, hi ? k : ok}, zd[2] = {hi ? od : d, hi ? d : od};
 #pragma unroll
   for (int z = 0; z < 2; ++z) {
     n[iu[z]] = fmax(n[iu[z]] - zd[z], R(0));
     n[iw[z]] += zd[z];
 #pragma unroll
-    for (int t2 = 0; t2 < LRP; ++t2) turn(x[iu[z]][t2], x[iw[z]][t2], zr[z], zi[z], zc[z]);
+    for (int t2 = 0; t2 < LRP; ++t2) turn(x[iu[z]][t2], x[iw[z]][t2], zr[z], zi[z], zk[z]);
   }
 }
 
@@ -283,6 +302,7 @@ __global__ __launch_bounds__(JAC_THREADS) void k_jacobi(JacArgs j, Ordering o) {
   C* A = reinterpret_cast<C*>(sm);                  // [q][PP]
   C* L = A + (size_t)q * PP;                        // [QP][LR]
   __shared__ C v0s[JAC_MAX_Q];
+  __shared__ double vh[JAC_MAX_Q], vl[JAC_MAX_Q];
   __shared__ R fs[JAC_MAX_Q], nrm[JAC_MAX_Q], red[JAC_THREADS / 64];
   __shared__ int pos[JAC_MAX_Q], busy[2], chi_s;
   __shared__ uint32_t lines[JAC_MAX_LINES];
@@ -363,8 +383,9 @@ __global__ __launch_bounds__(JAC_THREADS) void k_jacobi(JacArgs j, Ordering o) {
       if (c > k && c < q) {
 #pragma unroll
         for (int t = 0; t < RP; ++t) {
-          a[z][t].x = fma(-v[t].x, wr[z], fma(v[t].y, wi[z], a[z][t].x));
-          a[z][t].y = fma(-v[t].x, wi[z], fma(-v[t].y, wr[z], a[z][t].y));
+          // the change first: one rounding at the element's own size
+          a[z][t].x -= fma(v[t].x, wr[z], -v[t].y * wi[z]);
+          a[z][t].y -= fma(v[t].x, wi[z], v[t].y * wr[z]);
           A[c * PP + l + 16 * t] = a[z][t];
           if (to_l && l + 16 * t == k) {
             L[k * LR + c].x = a[z][t].x;
@@ -539,10 +560,12 @@ __global__ __launch_bounds__(JAC_THREADS) void k_jacobi(JacArgs j, Ordering o) {
   const int chi = chi_s;
   JacMeta* meta = reinterpret_cast<JacMeta*>(j.meta);
   if (tid < q) {
-    const double sg = (double)nrm[tid], rt = sqrt(ldexp(sg, ex));
+    const double sg = (double)nrm[tid], x = ldexp(sg, ex), rt = sqrt(x), rl = fma(-rt, rt, x) / (2 * rt);
     meta->pos[tid] = pos[tid];
     meta->root[tid] = rt;
-    fs[tid] = (R)(rt / sg);                         // V sqrt(sigma) = L x this
+    meta->rest[tid] = rl;
+    vh[tid] = rt / sg;                              // V sqrt(sigma) = L x (vh + vl)
+    vl[tid] = (fma(-vh[tid], sg, rt) + rl) / sg;
   }
   if (tid == 0) {
     meta->chi = chi;
@@ -554,10 +577,9 @@ __global__ __launch_bounds__(JAC_THREADS) void k_jacobi(JacArgs j, Ordering o) {
   for (int e = tid; e < q * q; e += JAC_THREADS) {
     const int c = e / q, r = e % q, at = pos[c];
     if (at >= chi) continue;
-    const R f = fs[c];
     C v = L[c * LR + r];
-    v.x *= f;
-    v.y *= j.trans ? f : -f;
+    v.x = times(v.x, vh[c], vl[c]);
+    v.y = times(j.trans ? v.y : -v.y, vh[c], vl[c]);
     out[j.trans ? r + (int64_t)j.m * at : at + (int64_t)chi * r] = v;
   }
 }
@@ -626,9 +648,9 @@ __global__ __launch_bounds__(64) void k_jacobi_left(JacArgs j, Ordering o) {
     const int at = meta->pos[c];
     if (at >= chi) continue;
     C v = buf[lr][c];
-    const R f = (R)meta->root[c];
-    v.x *= f;
-    v.y *= j.trans ? -f : f;
+    const double h = meta->root[c], l = meta->rest[c];
+    v.x = times(v.x, h, l);
+    v.y = times(j.trans ? -v.y : v.y, h, l);
     out[j.trans ? at + (int64_t)chi * row : row + (int64_t)j.m * at] = v;
   }
 }

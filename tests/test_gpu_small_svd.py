@@ -181,3 +181,47 @@ def test_zero_columns(ctx, m, n, zero, wide):
         ctx.profile_enable(False)
         assert copies == 0
         check(ctx, A, *got)
+
+
+def rounding_bound(n):
+    """Relative error of a split of n columns, in units of the roundoff u, if
+    every rotation and every reflection rounds an element once: at most 8
+    sweeps of n - 1 rotations on V Sigma and on U, 2 n reflections on U and R
+    and four more operations (scaling both factors), independent errors
+    uniform in +-u."""
+    return np.sqrt((2 * 8 * (n - 1) + 2 * n + 4) / 3)
+
+
+@pytest.mark.parametrize("m,n", [(8, 8), (16, 16), (20, 48), (64, 32), (32, 32), (64, 64)])
+def test_errors_grow_as_one_rounding_per_rotation(ctx, m, n):
+    """rms over matrices of |A - B C| / |A| in extended precision."""
+    rng = np.random.default_rng(m + n)
+    k, sq = min(m, n), []
+    for _ in range(max(4, 8192 // (m * n))):
+        u, w = np.linalg.qr(rnd(rng, m, k))[0], np.linalg.qr(rnd(rng, n, k))[0]
+        A = ((u * np.linspace(1, 0.1, k)) @ w.conj().T).astype(ctx.np_dtype).astype(np.clongdouble)
+        B, C, chi = split(ctx, A)
+        assert chi == k
+        d = (A - B.astype(np.clongdouble) @ C.astype(np.clongdouble)).astype(np.complex128)
+        sq.append((np.linalg.norm(d) / np.linalg.norm(A.astype(np.complex128))) ** 2)
+    assert np.sqrt(np.mean(sq)) <= rounding_bound(k) * np.finfo(ctx.np_dtype).eps / 2
+
+
+@pytest.mark.parametrize("m,n", [(4, 4), (12, 16), (32, 32), (64, 40), (64, 64)])
+def test_bond_dimension_beside_the_cutoff(ctx, m, n):
+    """Half the singular values lie beside the cut-off, in turn above and
+    below by twice four times the rounding error of a split: chi counts
+    exactly those above."""
+    rng = np.random.default_rng(7 * m + n)
+    k, eps = min(m, n), np.finfo(ctx.np_dtype).eps
+    cut = np.sqrt(eps)
+    near = 4 * rounding_bound(k) * eps / 2 / cut             # relative to the cut-off
+    s = np.linspace(1, 0.1, k)
+    head = k // 2
+    s[head:] = cut * np.linalg.norm(s[:head]) * (1 + 2 * near * np.where(np.arange(k - head) % 2, -1, 1))
+    u, w = np.linalg.qr(rnd(rng, m, k))[0], np.linalg.qr(rnd(rng, n, k))[0]
+    A = ((u * s) @ w.conj().T).astype(ctx.np_dtype).astype(np.complex128)
+    rel = np.linalg.svd(A, compute_uv=False)
+    rel /= np.linalg.norm(rel) * cut
+    assert np.all(np.abs(rel - 1) > near)                    # the input's own rounding moved none across
+    assert split(ctx, A)[2] == int(np.sum(rel > 1))
