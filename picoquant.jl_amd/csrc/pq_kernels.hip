@@ -44,8 +44,8 @@ __device__ __forceinline__ void store_one(C* p, const C& v) {
 // Bound: HBM, or the 256 MB last-level cache where X and Out fit it (7.6 TB/s
 // at 2^24 complex64).  NT: X and Out are together too large for that cache,
 // so Out (1) or both (2) pass it, and a lane takes one index instead of up
-// to 16 (launch_stream): 2^25 complex64 from three states in turn 117 -> 97
-// us, 2^26 195 -> 167.
+// to 16 (launch_stream has the rule): 2^25 complex64 from three states in turn
+// 117 -> 97 us, 2^26 195 -> 167.
 template <typename C, int KP, int NT>
 __global__ __launch_bounds__(256) void k_stream(const C* __restrict__ X, const C* __restrict__ Y,
                                                 C* __restrict__ Out, StreamArgs a) {
@@ -638,16 +638,35 @@ hipError_t launch_stream(const C* X, const C* Y, C* Out, const StreamArgs& a, hi
   int KP = 1;
   while ((uint32_t)KP < Kt) KP <<= 1;
   size_t smem = (size_t)KP * Nt * sizeof(C) + (size_t)Nt * 4;
-  // X and Out pass the caches when they are well over the last level's 256
-  // MB.  Measured a gate at a time, each on the last one's result: 256 MB
-  // together 35-43 us with the caches, 47-54 without; 512 MB 93-109 and
-  // 92-101; 1 GB 193-220 and 167-196.  X only where the lanes' loads cover its
-  // lines at once (the lowest bit summed, 512 MB: 97 us with X cached, 102
-  // without).  More than 4096 workgroups are an eighth slower where the
-  // caches serve (each stages Y) and a tenth faster past them.
-  const bool past = (double)a.M.total * a.L.total * (Kt + Nt) * sizeof(C) > 384.0 * (1 << 20);
-  const int nt = !past ? 0 : (a.M.m[0].s0 == 1 ? 2 : 1);
-  const dim3 grid(grid_for(a.M.total, 256, a.L.total > 1 ? 1024 : (past ? 65536 : 4096)), 1, a.L.total), block(256);
+  // X and Out together well over the last level's 256 MB pass the caches,
+  // Out or both, and a lane takes one index (or 64 bytes of X and Out), on up
+  // to 65536 workgroups.  Measured a gate at a time, each on the last one's
+  // result, us cached / Out passing / both passing, by the position of the
+  // bits summed:
+  //   complex64, 512 MB:  4 and 5 99 / 93 / 90, 1 and 9 99 / 92 / 95, 0 and 1
+  //     102 / 91 / 119, 0 to 2 110 / 107 / 183; 2 GB: 435 / 371 / 364, 433 /
+  //     369 / 389, 434 / 369 / 494, 442 / 404 / 733
+  //   complex128, 1 GB:  0 206 / 189 / 184, 1 and 9 206 / 209 / 200, 0 and 1
+  //     209 / 188 / 280, 5 to 7 206 / 219 / 203; 5 and 8 onto one 150 / 141 /
+  //     133; 512 MB: 0 97 / 97 / 93, 1 and 9 101 / 108 / 103, 0 and 1 105 / 96
+  //     / 143, 5 to 7 101 / 114 / 109
+  // so X passes only where its first mode runs over a whole 128-byte line (a
+  // shorter run is read by several loads, each fetching the line anew) or with
+  // two K values of 16 bytes.  complex128 stays cached from four K values on,
+  // unless Out is narrow or a lane's K values lie together; one index a lane
+  // still pays for four K values and 1 GB (1 and 9 206 -> 198, 2 GB 437 ->
+  // 397; eight K values 206 -> 213, 512 MB 101 -> 100 and up to 115).
+  // 256 MB together: 35-43 us cached, 47-54 passing.  Where the caches serve,
+  // more than 4096 workgroups are an eighth slower (each stages Y).
+  const double mb = (double)a.M.total * a.L.total * (Kt + Nt) * sizeof(C) / (1 << 20);
+  const bool line = a.M.nmodes > 0 && a.M.m[0].s0 == 1 && (uint64_t)a.M.m[0].ext.d * sizeof(C) >= 128;
+  const bool near = a.K.nmodes == 1 && a.K.m[0].s0 == 1;
+  int nt = 0;
+  if (mb > 384 && sizeof(C) == 8) nt = line ? 2 : 1;
+  if (mb > 384 && sizeof(C) == 16) nt = Kt <= 2 || (Nt <= 2 && line) ? 2 : (near ? 1 : 0);
+  const bool wide = nt != 0 || (mb > 640 && sizeof(C) == 16 && Kt <= 4 && Nt <= 4);
+  const uint64_t lanes = wide ? a.M.total / std::max<uint64_t>(64 / ((Kt + Nt) * sizeof(C)), 1) : a.M.total;
+  const dim3 grid(grid_for(lanes, 256, a.L.total > 1 ? 1024 : (wide ? 65536 : 4096)), 1, a.L.total), block(256);
   switch (KP * 4 + nt) {
 #define PQ_CASE2(P, NT) \
   case P * 4 + NT: hipLaunchKernelGGL((k_stream<C, P, NT>), grid, block, smem, s, X, Y, Out, a); break;

@@ -246,3 +246,33 @@ def test_stream_past_the_caches(ctx, K, N, k_first):
         x = x.astype(np.complex128)
         bound = (np.abs(y) @ np.abs(x)) * (2 * K + 4) * eps
         assert np.all(np.abs(got[:, m:m + (1 << 20)] - y @ x) <= bound)
+
+
+@pytest.mark.parametrize("run,K,N", [(1, 2, 2), (2, 4, 4), (4, 4, 2), (4, 8, 3), (7, 4, 1), (8, 2, 5), (8, 4, 4),
+                                     (15, 3, 4), (16, 4, 4), (16, 5, 2)])
+def test_stream_past_the_caches_runs(ctx, run, K, N):
+    """As above with the summed mode inside the operand: its first open mode
+    runs over less than a line, just a line or more."""
+    es = ctx.np_dtype.itemsize
+    rest = (400 << 20) // es // (K + N) // run | 1
+    rng = np.random.default_rng(run * 100 + K * 10 + N)
+    X = rng.random((rest, K, run, 2), dtype=np.float64 if es == 16 else np.float32)
+    X -= 0.5
+    X = X.view(ctx.np_dtype)[..., 0]                           # column-major [run, K, rest]
+    Y = rand(rng, (K, N), ctx.np_dtype)
+    hx, hy = ctx.upload(X.T), ctx.upload(Y)
+    ctx.set_kernel_override(_lib.KC_STREAM)
+    try:
+        hz = ctx.contract(hx, [-1, 1, -2], hy, [1, -3])
+    finally:
+        ctx.set_kernel_override(-1)
+    got = ctx.download(hz).T                                   # [N, rest, run]
+    for h in (hx, hy, hz):
+        ctx.free(h)
+    eps = 2.0 ** -53 if es == 16 else 2.0 ** -24
+    y = Y.T.astype(np.complex128)
+    step = max(1, (1 << 20) // run)
+    for m in range(0, rest, step):
+        x = X[m:m + step].transpose(1, 0, 2).reshape(K, -1).astype(np.complex128)
+        bound = (np.abs(y) @ np.abs(x)) * (2 * K + 4) * eps
+        assert np.all(np.abs(got[:, m:m + step].reshape(N, -1) - y @ x) <= bound)
