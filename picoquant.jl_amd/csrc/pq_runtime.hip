@@ -193,15 +193,25 @@ static C* dptr(const Tensor& t) {
 // six factors of two with the smallest input strides and the six with the
 // smallest output strides, so both sides move runs of 512 bytes or more
 // where the tensor has them, and the next output bits up to its size.  Not
-// for copies whose runs are long already (32 elements or more lie the same
-// way on both sides), small ones (below 2^15 elements the launch is the
-// cost), or where fewer factors of two exist than a tile has bits (odd
-// extents): k_copy takes those.
+// for small copies (below 8 MiB the launch and this function are the cost: 5.5
+// us by k_copy, 6.5 here), nor where fewer factors of two exist than a tile
+// has bits, nor where the tiles would touch more memory lines than k_copy's
+// lanes: a mode of odd extent lies outside the tile, and where one runs
+// fastest on a side, the tile's bits there are strides of it and every line is
+// read or written in parts by several workgroups.  Compared are the 128-byte
+// lines that 64 lanes touch, those written counted twice, the tile's times 1.5
+// (LDS) and k_copy's plus 1.5 for each mode it decodes.  Over 877 random
+// copies of both types, 2^15 to 2^24 elements, odd and even extents, this pick
+// is 1.01 times the faster of the two on average (1.9 at most; always tiles
+// 1.16 and 5.0, never 1.25 and 6.2).  us by k_copy / in tiles: complex128 [31,
+// 2048, 64] to [31, 64, 2048] 18.5 / 115, 4096 x 4099 turned 176 / 740, [64,
+// 3, 64, 5, 64] reordered 57 / 44, 48^4 reversed 66 / 23; complex64 [9, 512,
+// 3, 128] with its middle swapped 7 / 38, 2^24 bits in a random order 98 / 48.
 static bool copy_bits_args(const std::vector<Mode>& modes, size_t esize, CopyBitsArgs& a) {
   const int nb = CB_BITS(esize);
   int64_t total = 1;
   for (const Mode& m : modes) total *= m.ext;
-  if (total < (1 << 15) || modes.empty() || (modes[0].s0 == 1 && modes[0].ext >= 32)) return false;
+  if (total * (int64_t)esize < (8 << 20) || modes.empty()) return false;
   struct Bit {
     int64_t in, out;
     int mode, tile;
@@ -250,6 +260,38 @@ static bool copy_bits_args(const std::vector<Mode>& modes, size_t esize, CopyBit
       used |= 1u << f;
       vec[lo[k]] |= 1 << f;
     }
+  // lines of 64 lanes: the tile's loads and stores, k_copy's loads (its
+  // stores run on)
+  auto lines = [&](const int64_t (&o)[64]) {       // distinct ones, by a table of 128 slots
+    int64_t slot[128];
+    uint64_t used[2] = {0, 0};
+    int n = 0;
+    for (int64_t x : o) {
+      x = (uint64_t)x * esize >> 7;
+      unsigned h = (unsigned)((uint64_t)x * 0x9e3779b97f4a7c15ull >> 57);
+      for (; (used[h >> 6] >> (h & 63)) & 1; h = (h + 1) & 127)
+        if (slot[h] == x) break;
+      if ((used[h >> 6] >> (h & 63)) & 1) continue;
+      used[h >> 6] |= 1ull << (h & 63);
+      slot[h] = x;
+      ++n;
+    }
+    return n;
+  };
+  int64_t tl[64] = {0}, ts[64] = {0}, kl[64];
+  for (int i = 1; i < 64; ++i) {
+    const int top = 31 - __builtin_clz((unsigned)i);
+    tl[i] = tl[i ^ (1 << top)] + bits[li[top]].in;
+    ts[i] = ts[i ^ (1 << top)] + bits[lo[top]].out;
+  }
+  int done = 1;                                    // lanes whose place is known, by mode
+  kl[0] = 0;
+  for (size_t q = 0; q < modes.size() && done < 64; ++q) {
+    const int step = done;
+    for (; done < 64 && done < step * modes[q].ext; ++done) kl[done] = kl[done - step] + modes[q].s0;
+  }
+  const double tiled = 1.5 * (lines(tl) + 2 * lines(ts));
+  if (tiled >= lines(kl) + 2 * (int)(64 * esize / 128) + 1.5 * modes.size()) return false;
   memset(&a, 0, sizeof(a));
   for (int k = 0; k < nb; ++k) {
     a.is[k] = (int32_t)bits[li[k]].in;

@@ -72,3 +72,18 @@ def test_past_the_caches(ctx):
     an odd factor among the extents."""
     dims = [2] * 22 + ([5] if ctx.np_dtype == np.complex128 else [2, 5])
     check(ctx, dims, np.random.default_rng(len(dims)).permutation(len(dims)).tolist())
+
+
+@pytest.mark.parametrize("dims,perm", [
+    ([31, 2048, 32], [0, 2, 1]), ([2048, 1025], [1, 0]), ([1025, 2048], [1, 0]),    # an odd extent fastest
+    ([64, 64, 64, 7], [3, 0, 1, 2]), ([9, 512, 3, 128], [0, 2, 1, 3]),
+    ([64, 3, 64, 3, 64], [1, 4, 3, 0, 2]), ([48, 48, 48, 20], [3, 2, 1, 0]), ([7, 64, 64, 64], [3, 2, 1, 0]),
+    ([3, 1024, 512], [2, 1, 0]), ([12, 24, 36, 16, 8], [4, 2, 0, 3, 1]), ([16, 65536, 2], [1, 0, 2]),
+    ([24, 2048, 32], [0, 2, 1]), ([2] * 9 + [3] + [2] * 11, [20, 3, 1, 19, 9, 0, 18, 2, 17, 4, 16, 5, 15, 6, 14, 7, 13, 8, 12, 10, 11]),
+    ([2] * 21, [0, 1, 2, 3] + list(range(20, 3, -1))), ([128, 2, 31, 96, 3], [2, 1, 4, 3, 0])])
+def test_odd_extents_beside_factors_of_two(ctx, dims, perm):
+    """Copies over the size where tiles begin, whose odd extents keep them out
+    of tiles or run beside them, and a slice of each."""
+    check(ctx, dims, perm)
+    n = dims[perm[0]]
+    check(ctx, dims, perm, (1, n // 2 + 1, n))
