@@ -197,9 +197,10 @@ typedef struct {
   int32_t n_slots;
   const int64_t* slot_elems;        /* per-slice elements (leaves: all elements) */
   const int64_t* slot_batch_mask;   /* bit j set: the slot holds one copy per value of sliced
-                                       bond j within a slice group (for j < group_bits) and is
-                                       recomputed per slice group (j >= group_bits); 0 = the
-                                       slot does not depend on any sliced bond */
+                                       bond j within a slice group (j < group_bits, and the
+                                       output-batch bonds that join it, see budget_bytes) and is
+                                       recomputed per slice group (the other j); 0 = the slot does
+                                       not depend on any sliced bond */
   const pq_tensor* slot_leaf;       /* leaf tensor, 0 for intermediates */
   int32_t n_sliced;                 /* number of sliced bonds (extent 2 each) */
   const int64_t* slot_slice_stride; /* [n_slots * n_sliced] stride of sliced bond j in an unbatched
@@ -240,7 +241,14 @@ typedef struct {
                                        vector for bitstring b ([1, 0] for 0, [0, 1] for 1,
                                        src/layer3.jl:292-313) */
   const int32_t* out_qubit_bit;     /* [n_out_qubits] the qubit's bit in a bitstring word (0-63) */
+  int64_t budget_bytes;             /* with n_out_bits > 0 and every other sliced bond in the slice
+                                       group, output-batch bonds join the group while no tensor's
+                                       copies exceed PQ_OUT_GROUP_SLOT_BYTES and the plan's arena and
+                                       scratch together neither PQ_OUT_GROUP_BYTES nor this (0: no
+                                       further limit); the rest run one group after another */
 } pq_plan_desc;
+#define PQ_OUT_GROUP_SLOT_BYTES ((int64_t)256 << 20)
+#define PQ_OUT_GROUP_BYTES ((int64_t)1 << 30)
 
 /* A fused chain applies L small complex64 operators one after the other to
  * one large complex64 tensor, as L contraction steps would (each step sums

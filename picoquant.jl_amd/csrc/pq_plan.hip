@@ -861,19 +861,19 @@ int run_program(pq_ctx* c, pq_plan* p, bool profile_steps) {
   return PQ_OK;
 }
 
-// Output-batch bonds that join the slice group: a batch of bitstrings then
-// runs as more copies of each batched step (grid z, or extra rows of a
-// product whose other operand no bitstring changes) instead of once more
-// through the launch sequence per bitstring.  A launch is worth the batch
-// while its tensors are small: 64 ComplexF64 amplitudes of the 5x5
-// depth-12 grid circuit (peak 2^18 elements) took 17.2 ms as 64 groups of
-// launches of 4-23 us each, and take 1.70 ms in one group.  The copies of
-// every intermediate stay within OUT_GROUP_BYTES, the size of the last-level
-// cache (16 / 64 / 1024 MiB on that plan: 6.23 / 2.67 / 1.69 ms; the limit
-// also keeps every stride far below 2^31), a group has at most
-// PQ_MAX_BMODES bits, and plans whose fused chains depend on the bitstrings
-// keep one group per bitstring (a chain runs once per group).
-#define OUT_GROUP_BYTES ((int64_t)256 << 20)
+// Most output-batch bonds that may join the slice group: a batch of
+// bitstrings then runs as more copies of each batched step (grid z, or extra
+// rows of a product whose other operand no bitstring changes) instead of once
+// more through the launch sequence per bitstring.  A launch is worth the batch
+// while its tensors are small: 64 ComplexF64 amplitudes of the 5x5 depth-12
+// grid circuit (peak 2^18 elements) took 17.2 ms as 64 groups of launches of
+// 4-23 us each, and take 0.94 ms in one group.  The copies of every
+// intermediate stay within PQ_OUT_GROUP_SLOT_BYTES, the size of the last-level
+// cache (with 16 / 64 / 1024 MiB that plan, when it took 1.69 ms, took 6.23 /
+// 2.67 / 1.69; the limit also keeps every stride far below 2^31), the plan
+// within PQ_OUT_GROUP_BYTES and the caller's budget (create_plan), a group has
+// at most PQ_MAX_BMODES bits, and plans whose fused chains depend on the
+// bitstrings keep one group per bitstring (a chain runs once per group).
 int out_bits_in_group(const pq_ctx* c, const pq_plan_desc* d) {
   if (d->n_slots <= 0 || d->n_steps < 0 || d->n_sliced < 0 || d->n_sliced > 40 || d->group_bits < 0 ||
       d->n_out_bits < 1 || d->n_out_bits > d->n_sliced || d->group_bits != d->n_sliced - d->n_out_bits ||
@@ -893,7 +893,7 @@ int out_bits_in_group(const pq_ctx* c, const pq_plan_desc* d) {
       const int64_t es = (d->slot_dtype ? d->slot_dtype[s] : c->dtype) == PQ_C128 ? 16 : 8;
       if (low >> d->group_bits)
         fits = d->slot_elems[s] > 0 &&
-               d->slot_elems[s] <= (OUT_GROUP_BYTES / es) >> __builtin_popcountll(low);
+               d->slot_elems[s] <= (PQ_OUT_GROUP_SLOT_BYTES / es) >> __builtin_popcountll(low);
     }
     if (fits) break;
   }
@@ -1327,6 +1327,14 @@ int create_plan(pq_ctx* c, const pq_plan_desc* d, int out_in_group, pq_plan** ou
   }
   p->arena_bytes = std::max<size_t>(top, 256);
   p->out_elems = p->slots[p->out_slot].elems;
+  if (out_in_group > 0) {
+    int64_t most = PQ_OUT_GROUP_BYTES;
+    if (d->budget_bytes > 0) most = std::min(most, d->budget_bytes);
+    if (p->arena_bytes + p->scratch_bytes > (size_t)most) {
+      free_plan(c, p);
+      return fail(c, PQ_ERR_OOM, "output batches in the slice group exceed the budget");
+    }
+  }
   if (hipMalloc(&p->arena, p->arena_bytes) != hipSuccess ||
       (p->scratch_bytes && hipMalloc(&p->scratch, p->scratch_bytes) != hipSuccess) ||
       hipMalloc((void**)&p->out_dev, sizeof(double) * 2 * p->out_elems * p->n_out) != hipSuccess) {
@@ -1649,10 +1657,10 @@ extern "C" {
 
 int pq_plan_create(pq_ctx* c, const pq_plan_desc* d, pq_plan** out) {
   if (!c || !d || !out) return PQ_ERR_ARG;
-  const int e = out_bits_in_group(c, d);
-  // a plan that cannot be built with its output batches in the slice group
-  // (memory, launch limits) runs them one after another
-  if (e > 0 && create_plan(c, d, e, out) == PQ_OK) return PQ_OK;
+  // a plan that cannot be built with so many output batches in the slice
+  // group (memory, launch limits) runs more of them one after another
+  for (int e = out_bits_in_group(c, d); e > 0; --e)
+    if (create_plan(c, d, e, out) == PQ_OK) return PQ_OK;
   return create_plan(c, d, 0, out);
 }
 

@@ -53,6 +53,7 @@ class PlanDesc(ct.Structure):
         ("n_out_qubits", ct.c_int32),
         ("out_qubit_slot", ct.POINTER(ct.c_int32)),
         ("out_qubit_bit", ct.POINTER(ct.c_int32)),
+        ("budget_bytes", ct.c_int64),
     ]
 
 
@@ -779,6 +780,8 @@ def compile_plan(network, plan, sliced=(), out_order=None, group_bits=None, kc=N
     `plan` (kernel class and GEMM tile, -1 = automatic).  fuse: runs of
     complex64 steps that apply small operators to one large tensor become
     fused-chain steps (fuse_chains; a dict passes its limits).
+    budget_bytes: device memory for the intermediates of a slice group (when
+    group_bits is not given) and for a bitstring batch's joining it.
     bitstrings: a batch of output bitstrings (output_batch) computed in one
     run, one result per bitstring; the closed output qubits' leaves are
     replaced by device tensors with a column per bitstring, which
@@ -859,7 +862,8 @@ def compile_plan(network, plan, sliced=(), out_order=None, group_bits=None, kc=N
     d = PlanDesc(len(slots), keep["slot_elems"], keep["slot_mask"], keep["slot_leaf"], n_sliced, keep["lss"],
                  group_bits, len(steps), keep["step_slots"], keep["kc"], keep["tile"], keep["nmodes"],
                  keep["modes"], out_slot, keep["dt"], keep["kind"], keep["arith"], keep["chain_off"],
-                 len(words), keep["words"], n_out_bits, len(oq_slot), keep["oq_slot"], keep["oq_bit"])
+                 len(words), keep["words"], n_out_bits, len(oq_slot), keep["oq_slot"], keep["oq_bit"],
+                 int(max(1, min(budget_bytes, 1 << 62))))
     p = ct.c_void_p()
     try:
         ctx.check(ctx.lib.pq_plan_create(ctx.ptr, ct.cast(ct.pointer(d), ct.c_void_p), ct.byref(p)))

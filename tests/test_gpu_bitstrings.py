@@ -208,3 +208,33 @@ def test_bitstring_batch_inside_the_slice_group(n_sliced, group_bits, precision,
         want = np.array([[_amp(sv, list(b.replace("x", v))) for v in "01"] for b in batch])
         assert np.max(np.abs(got - want)) <= (1e-12 if precision == "uniform" else 1e-5) * np.max(np.abs(want))
     p.close()
+
+
+def test_bitstring_batch_keeps_to_the_budget():
+    """budget_bytes bounds the plan's memory with bitstrings inside the slice
+    group: less of it, fewer join, down to one group per bitstring; any
+    number that compile_plan took before is taken (0, floats, infinity)."""
+    n, count = 12, 32
+    sv = O.statevector(n, O.grid_circuit_gates(3, 4, 8, 5))
+    rng = np.random.default_rng(2)
+    batch = ["".join(str(int(v)) for v in rng.integers(0, 2, n)) for _ in range(count)]
+    want = np.array([_amp(sv, list(b)) for b in batch])
+    tn = _net(3, 4, 8, 5, batch[0])
+    plan = PL.sweep_plan(tn, PL.grid_site_order(3, 4))
+
+    def run(**kw):
+        p = compile_plan(tn, plan, bitstrings=batch, **kw)
+        st = p.stats()
+        assert np.max(np.abs(p.run(batch) - want)) <= 1e-12 * np.max(np.abs(want))
+        p.close()
+        return st["arena_bytes"], st["launches"]
+
+    full, one = run(), run(budget_bytes=0)
+    assert run(budget_bytes=float("inf")) == full
+    assert full[0] > one[0] and full[1] < one[1]
+    last = full
+    for budget in (full[0] - 1, (full[0] + one[0]) / 2, one[0]):
+        got = run(budget_bytes=budget)
+        assert got[0] <= budget and got[1] >= last[1] and got != full
+        last = got
+    assert run(budget_bytes=one[0] - 1) == one
