@@ -45,7 +45,11 @@ int pq_ctx_dtype(const pq_ctx* ctx);
 int pq_synchronize(pq_ctx* ctx);
 
 /* save_tensor_data: store a converted copy (src/backends/interactive.jl:32-36).
- * host_dtype (PQ_C128 / PQ_C64) is converted to the context's element type. */
+ * host_dtype (PQ_C128 / PQ_C64) is converted to the context's element type.
+ * The host buffer may be reused on return.  Data of at most 1 KiB (in the
+ * context's type) travels in a kernel's arguments and is not waited for: it
+ * is stream-ordered before later work on the context, and a failure of that
+ * or earlier work is reported by a later call; larger data is synchronised. */
 int pq_tensor_upload(pq_ctx* ctx, int rank, const int64_t* dims, const void* host,
                      int host_dtype, pq_tensor* out);
 
@@ -127,7 +131,11 @@ int pq_decompose(pq_ctx* ctx, pq_tensor t, int nleft, const int32_t* left, int n
                  double threshold, int max_rank, pq_tensor* B, pq_tensor* C, int* chi);
 
 /* Device pointer and element offset of a tensor (for in-process callers that
- * share device memory, e.g. tests comparing against torch). */
+ * share device memory, e.g. tests comparing against torch).  Synchronises the
+ * context's stream if small uploads or bitstrings were written since the last
+ * call, so that host data is there for any stream; results of contractions
+ * and plans are stream-ordered (pq_synchronize before reading them from
+ * another stream). */
 int pq_tensor_device_ptr(pq_ctx* ctx, pq_tensor t, void** base, int64_t* elem_offset,
                          int64_t* strides);
 
@@ -311,8 +319,8 @@ int pq_plan_cost(const pq_plan* plan, pq_cost* total, double* step_macs, double*
  * qubit q takes (the reference's add_output! per bitstring,
  * src/layer3.jl:292-313).  1 <= n_bitstrings <= 2^n_out_bits; a shorter
  * batch is padded with copies of the first bitstring.  Rewrites the qubits'
- * leaves in place (stream-ordered before later runs), so a captured graph
- * computes the new batch on its next replay. */
+ * leaves in place (stream-ordered before later runs, not waited for), so a
+ * captured graph computes the new batch on its next replay. */
 int pq_plan_set_bitstrings(pq_ctx* ctx, pq_plan* plan, int n_bitstrings, const uint64_t* bitstrings);
 /* One call for the batched path: the bitstrings (if n_bitstrings > 0), one
  * graph-replayed run over every slice, and the FP64 result into out_fp64

@@ -1796,6 +1796,7 @@ int pq_plan_set_bitstrings(pq_ctx* c, pq_plan* p, int n, const uint64_t* bits) {
   const int64_t nb = (int64_t)1 << p->n_out_bits;
   if (n < 1 || (int64_t)n > nb || !bits) return fail(c, PQ_ERR_ARG, "bitstring count out of range");
   BitWords words;
+  c->unsynced = true;
   for (int64_t first = 0; first < nb; first += SET_BITS_WORDS) {
     const int m = (int)std::min<int64_t>(nb - first, SET_BITS_WORDS);
     for (int t = 0; t < m; ++t) words.w[t] = bits[first + t < n ? first + t : 0];

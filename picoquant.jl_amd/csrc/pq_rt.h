@@ -75,7 +75,7 @@ struct pq_ctx {
   std::multimap<size_t, void*> free_blocks;
   size_t cached = 0;
   bool prof = false;
-  bool unsynced = false;    // uploads not waited for (pq_tensor_upload's small ones)
+  bool unsynced = false;    // host data written and not waited for (small uploads, bitstrings)
   bool capturing = false;
   pqrt::ProfEntry pe[PQ_KC_COUNT];
   int override_kc = -1;

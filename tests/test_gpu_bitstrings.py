@@ -21,7 +21,7 @@ import pytest
 from oracle import pq_oracle as O
 import picoquant_hip as P
 from picoquant_hip import _lib, circuits as C, planner as PL
-from picoquant_hip.executor import compile_plan
+from picoquant_hip.executor import closed_output_qubits, compile_plan
 
 pytestmark = pytest.mark.gpu
 
@@ -238,3 +238,49 @@ def test_bitstring_batch_keeps_to_the_budget():
         assert got[0] <= budget and got[1] >= last[1] and got != full
         last = got
     assert run(budget_bytes=one[0] - 1) == one
+
+
+def test_rewritten_bitstrings_are_there_for_other_streams():
+    """pq_tensor_device_ptr of an output column, taken after set_bitstrings
+    behind 10 ms of queued work, is safe to read from another stream."""
+    import ctypes as ct
+    n = 4
+    rng = np.random.default_rng(3)
+    batches = [["".join(str(int(v)) for v in rng.integers(0, 2, n)) for _ in range(8)] for _ in range(2)]
+    tn = _net(2, 2, 3, 5, batches[0][0])
+    p = compile_plan(tn, PL.sweep_plan(tn, PL.grid_site_order(2, 2)), bitstrings=batches[0])
+    ctx, hip = p.ctx, p.ctx.lib                            # the HIP runtime, through the library that links it
+    stream = ct.c_void_p()
+    assert hip.hipStreamCreateWithFlags(ct.byref(stream), ct.c_uint(1)) == 0        # does not wait for others
+    cols = {}
+
+    def read(where):
+        for qubit, src in where.items():
+            out = np.empty((8, 2), np.complex128)
+            assert hip.hipMemcpyAsync(ct.c_void_p(out.ctypes.data), ct.c_void_p(src), ct.c_size_t(out.nbytes),
+                                      ct.c_int(2), stream) == 0
+            assert hip.hipStreamSynchronize(stream) == 0
+            cols[qubit] = out
+
+    def pointers():
+        base, off, where = ct.c_void_p(), ct.c_int64(), {}
+        for node, qubit in closed_output_qubits(tn):
+            ctx.check(hip.pq_tensor_device_ptr(ctx.ptr, p.batch_handles[node], ct.byref(base), ct.byref(off), None))
+            where[qubit] = base.value + 16 * off.value
+        return where
+
+    read(pointers())                                       # the copies' own first use
+    big = ctx.upload(np.ones((4096, 4096), np.complex128))
+    first = ctx.contract(big, [-1, 1], big, [1, -2])       # memory and kernels are there
+    ctx.synchronize()
+    ctx.free(first)
+    busy = ctx.contract(big, [-1, 1], big, [1, -2])
+    p.set_bitstrings(batches[1])
+    read(pointers())
+    for qubit, col in cols.items():
+        assert np.array_equal(col, [[1 - int(b[qubit]), int(b[qubit])] for b in batches[1]])
+    ctx.synchronize()
+    hip.hipStreamDestroy(stream)
+    ctx.free(busy)
+    ctx.free(big)
+    p.close()
