@@ -123,8 +123,11 @@ int pq_materialize(pq_ctx* ctx, pq_tensor t, pq_tensor* out);
  * spectrum's 2-norm exceeds max(threshold, sqrt(eps)) of the element type,
  * capped by max_rank when max_rank > 0.  t is not consumed (the caller
  * frees it, as the backend verb does).  On the GPU: one-sided Jacobi in two
- * launches when the shorter side is at most 64 and the longer fits one
- * workgroup's LDS (256 for a shorter side of 32), else rocSOLVER gesdd;
+ * launches when the shorter side is at most 64 and the longer at most 256 and
+ * fits one workgroup's LDS (128 for a shorter side of 33 to 44 in complex128
+ * or 61 to 64 in complex64, 64 for 45 to 64 in complex128; both sides together
+ * 256 for a shorter side of up to 4 in complex128 or 5 to 8 in complex64, 128
+ * for up to 4 in complex64), else rocSOLVER gesdd;
  * synchronises the context's stream (chi is needed on the host).  A tensor
  * with no singular value above the threshold gives PQ_ERR_UNSUPPORTED. */
 int pq_decompose(pq_ctx* ctx, pq_tensor t, int nleft, const int32_t* left, int nright, const int32_t* right,

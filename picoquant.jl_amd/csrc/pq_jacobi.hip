@@ -692,7 +692,8 @@ size_t lds_bytes(int p, int q, size_t es) {
 bool jacobi_fits(int64_t m, int64_t n, size_t es) {
   const int64_t p = std::max(m, n), q = std::min(m, n);
   if (q < 1 || q > JAC_MAX_Q || p > 256) return false;
-  // the offsets of X's rows and columns pass through L
+  // the offsets of X's rows and columns pass through L, which is small for few
+  // columns
   const int qp = pad_q((int)q);
   if ((size_t)(m + n) * 4 > (size_t)qp * std::max(qp, 16) * es) return false;
   return lds_bytes((int)p, (int)q, es) <= JAC_LDS_BYTES;

@@ -225,3 +225,22 @@ def test_bond_dimension_beside_the_cutoff(ctx, m, n):
     rel /= np.linalg.norm(rel) * cut
     assert np.all(np.abs(rel - 1) > near)                    # the input's own rounding moved none across
     assert split(ctx, A)[2] == int(np.sum(rel > 1))
+
+
+@pytest.mark.parametrize("shorter,longer", [(1, (255, 127)), (4, (252, 124)), (5, (256, 251)), (8, (256, 248)),
+                                            (9, (256, 256)), (32, (256, 256)), (33, (128, 256)), (44, (128, 256)),
+                                            (45, (64, 256)), (60, (64, 256)), (61, (64, 128)), (64, (64, 128))])
+def test_size_rule(ctx, shorter, longer):
+    """The longest matrix (complex128, complex64) that the kernel takes, and
+    one row or column more, which the library takes (its path starts with a
+    copy, which the profile counts)."""
+    rng = np.random.default_rng(shorter)
+    most = longer[0 if ctx.np_dtype == np.complex128 else 1]
+    for m, n, copied in ((most, shorter, 0), (shorter, most, 0), (most + 1, shorter, 1), (shorter, most + 1, 1)):
+        A = rnd(rng, m, n).astype(ctx.np_dtype).astype(np.complex128)
+        ctx.profile_enable(True)
+        got = split(ctx, A)
+        copies = ctx.profile_read(_lib.KC_COPY)["launches"]
+        ctx.profile_enable(False)
+        assert copies == copied, (m, n)
+        check(ctx, A, *got)
