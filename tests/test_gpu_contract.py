@@ -276,3 +276,18 @@ def test_stream_past_the_caches_runs(ctx, run, K, N):
         x = X[m:m + step].transpose(1, 0, 2).reshape(K, -1).astype(np.complex128)
         bound = (np.abs(y) @ np.abs(x)) * (2 * K + 4) * eps
         assert np.all(np.abs(got[:, m:m + step].reshape(N, -1) - y @ x) <= bound)
+
+
+@pytest.mark.parametrize("M,N,K", [(7, 6, (301,)), (5, 3, ()), (9, 4, (1,)), (3, 17, (2, 3)), (4, 5, (5, 2, 7)),
+                                   (13, 11, (2, 2, 2, 2, 2, 2)), (300, 2, (3, 4)), (2, 3, (4, 9, 3, 5))])
+@pytest.mark.parametrize("flip", [False, True])
+def test_generic_sums_along_runs(ctx, M, N, K, flip):
+    """The serial kernel over summed modes of every number and run length,
+    in the same order in both tensors (one run) and reversed (many)."""
+    rng = np.random.default_rng(M + N + sum(K))
+    q = len(K)
+    A = rand(rng, (M,) + K, ctx.np_dtype)
+    order = list(range(q))[::-1] if flip else list(range(q))
+    B = rand(rng, tuple(K[i] for i in order) + (N,), ctx.np_dtype)
+    ia, ib = [-1] + [i + 1 for i in range(q)], [i + 1 for i in order] + [-2]
+    check(ctx, A, ia, B, ib, run(ctx, A, ia, B, ib, _lib.KC_GENERIC))
