@@ -112,8 +112,9 @@ __device__ __forceinline__ void group_offsets(const Group& g, uint32_t i, int32_
 // start of a kernel: met one by one by the decoding loops, each is a wait of
 // its own for memory the launch has just written.  With the modes' fields
 // together and power-of-two extents decoded by shifts, a two-qubit gate on 12
-// qubits takes 3.8 us on the device instead of 5.9, and replays of the 5x5 /
-// 6x6 / 7x7 grid plans 901 / 1119 / 787 us instead of 962 / 1157 / 856.
+// qubits takes 3.4 us on the device instead of 5.0 (2000 in a row; its call is
+// bound by the host either way), and replays of the 5x5 / 6x6 / 7x7 grid plans
+// 901 / 1119 / 787 us instead of 962 / 1157 / 856.
 #define PQ_TOUCH(G0, G1, G2, L0)                                                                             \
   asm volatile("" ::"s"((G0).nmodes), "s"((G0).m[0].s1), "s"((G0).m[2].s1), "s"((G1).nmodes),                 \
                "s"((G1).m[0].s1), "s"((G1).m[2].s1), "s"((G2).nmodes), "s"((G2).m[0].s1), "s"((G2).m[2].s1), \

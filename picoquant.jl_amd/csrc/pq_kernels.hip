@@ -360,8 +360,9 @@ __global__ __launch_bounds__(PQ_PUT_WORDS) void k_put(uint32_t* __restrict__ dst
 // Bound: HBM (2^24 complex64 elements in a random axis order: 48 us = 5.5
 // TB/s, 107 us by k_copy, whose time is its per-element decode).  NT: In and
 // Out are together well over the 256 MB last-level cache and Out passes it
-// (2^24 complex128, three tensors in turn 109 -> 104 us and 107 -> 98, one
-// again and again 121 -> 80).
+// (2^24 complex128 in six random orders: three tensors in turn 103-126 us
+// cached, 97-126 past it, one of them slower; one again and again 101-126 and
+// 67-76).
 template <typename C, bool NT>
 __global__ __launch_bounds__(256) void k_copy_bits(const C* __restrict__ In, C* __restrict__ Out, CopyBitsArgs a) {
   constexpr int NB = CB_BITS(sizeof(C)), PER = 1 << (NB - 8);
